@@ -264,6 +264,12 @@ int set_tiling(dg_ctx *c, int tile_y, int chunk_x)
     return DG_OK;
 }
 
+static DivConst div_const(float b)
+{
+    const double bd = b, h = 1.0 / bd;
+    return {h, std::fma(-bd, h, 1.0) * h};
+}
+
 // Validates a configuration and derives the kernel arguments (grid,
 // boundaries, constants, default tiling) from it.
 int make_args(const dg_config *cfg, StepArgs *out, int *tile_y_out, int *heat_mask_out, std::string *why)
@@ -294,11 +300,11 @@ int make_args(const dg_config *cfg, StepArgs *out, int *tile_y_out, int *heat_ma
     const size_t el_bytes = cfg->precision == DG_FP64 ? sizeof(double) : sizeof(float);
     if (n3 * el_bytes >= ((size_t)1 << 32)) return bad("a field of this grid exceeds 4 GiB");
     const int prec = cfg->precision, fast = cfg->math == DG_MATH_FAST;
-    // default tile height: 8 rows (two workgroups per CU); FP32 exact math
-    // keeps one 16-row workgroup per CU (its register footprint allows no
-    // second one, and the taller tile re-reads fewer halo rows): 29.8 against
-    // 25.6 Gcell/s on a 512^3 periodic grid
-    int ty = cfg->tile_y ? cfg->tile_y : ((prec == DG_FP32 && !fast) ? 16 : 8);
+    // default tile height: 8 rows (two workgroups per CU); FP32 exact math, bound
+    // by its VALU work, takes one 16-row workgroup per CU (fewer halo states per
+    // cell): KHI 512^3 38.9 against 36.0 Gcell/s at 8 rows, FP32-bulk minmod
+    // 256^3 34.3 against 32.3
+    int ty = cfg->tile_y ? cfg->tile_y : ((prec != DG_FP64 && !fast) ? 16 : 8);
     if (prec == DG_FP64 && ty > 8) ty = 8;
 
     StepArgs a{};
@@ -321,6 +327,14 @@ int make_args(const dg_config *cfg, StepArgs *out, int *tile_y_out, int *heat_ma
     }
     a.gamma = cfg->gamma;
     a.g = cfg->g;
+    {
+        // the divisors of the FP32 exact kernels, in the kernels' float arithmetic
+        const float ds = (float)cfg->ds, V = ds * ds * ds;
+        a.dV = div_const(V);
+        a.dgm1 = div_const((float)cfg->gamma - 1.0f);
+        a.d2ds = div_const(2.0f * ds);
+        a.dds = div_const(ds);
+    }
     if (tile_args(a, prec, ty, cfg->chunk_x, nullptr) != DG_OK) return bad("invalid tile_y or chunk_x");
     *out = a;
     if (tile_y_out) *tile_y_out = ty;

@@ -17,6 +17,9 @@ enum : int { LIM_NONE = 0, LIM_MINMOD = 1, LIM_VANLEER = 2 };
 // the step kernel, which does not accumulate them).
 constexpr int PARTIAL_STRIDE = 8;
 
+// A constant FP32 divisor b as 1 / b = h + l (exact_div, dg_step.hip).
+struct DivConst { double h, l; };
+
 struct StepArgs {
     int n[3];          // interior cells per axis
     int bc[6];         // x-, x+, y-, y+, z-, z+
@@ -29,6 +32,7 @@ struct StepArgs {
     int pow2;          // 1: ds is a power of two, so x / ds, x / (2 ds) and x / ds^3
                        //    equal the products with the exact reciprocals bit for bit
     double ds, gamma, g;
+    DivConst dV, dgm1, d2ds, dds;   // ds^3, gamma - 1, 2 ds, ds (in float arithmetic)
 };
 
 // Device-resident scalars of a context.

@@ -81,6 +81,74 @@ template <typename T> __device__ __forceinline__ T dsqrt_fast(T x);
 template <> __device__ __forceinline__ float dsqrt_fast<float>(float x) { return __builtin_amdgcn_sqrtf(x); }
 template <> __device__ __forceinline__ double dsqrt_fast<double>(double x) { return sqrt(x); }
 
+// ---- IEEE division and square root for the exact kernels --
+// The compiler's correctly rounded FP32 division costs ~12 issue slots (two
+// v_div_scale, a reciprocal, six fused operations, v_div_fmas, v_div_fixup)
+// and every division pays it in full, though the scheme divides several
+// numbers by the same one (a face's star density, a cell's mass) and many by
+// constants.  Here a float divisor becomes 1 / b = h + l in FP64 once (10
+// slots; 0 for a constant) and each quotient is one FP64 product rounded to
+// float (5 slots; FP64 multiplies, FMAs and conversions issue at the FP32
+// rate on this chip, 4.4-4.8 cycles measured, v_rcp_f64 16).  The result is
+// the correctly rounded quotient: a / b of two 24-bit numbers lies at least
+// 2^-49 |a / b| away from every rounding boundary it is not equal to (a - b m
+// is a nonzero multiple of the product of the last places), and the FP64
+// value is within 2^-53; a quotient that FP64 holds exactly, a tie between
+// two denormals included, comes out exactly, since a (h + l) is a / b within
+// 2^-100 and rounded once.  v_div_fixup sets zeros, infinities, NaNs and
+// signs as the compiled division does.
+template <typename T> struct Divisor;
+template <> struct Divisor<float> { float b; double h, l; };
+__device__ __forceinline__ Divisor<float> make_divisor(float b)
+{
+    const double bd = b, y = __builtin_amdgcn_rcp(bd);       // ~2^-24
+    const double e = fma(-bd, y, 1.0);
+    const double h = fma(y, fma(e, e, e), y);                // 1 / b to FP64 rounding (error e^3 before it)
+    return {b, h, fma(-bd, h, 1.0) * h};
+}
+__device__ __forceinline__ float exact_div(float a, const Divisor<float> &D)
+{
+    const double ad = a;
+    return __builtin_amdgcn_div_fixupf((float)fma(ad, D.h, ad * D.l), D.b, a);
+}
+// 1 / b: h alone is enough (a tie would need b and 1 / b both powers of two)
+__device__ __forceinline__ float exact_rcp(float b)
+{
+    const double bd = b, y = __builtin_amdgcn_rcp(bd);
+    const double e = fma(-bd, y, 1.0);
+    return __builtin_amdgcn_div_fixupf((float)fma(y, fma(e, e, e), y), b, 1.0f);
+}
+// sqrt(x / r), both correctly rounded.  A quotient of at least 2^-96 (not
+// NaN, zero or negative) takes the short path: the quotient as above, its
+// square root as the hardware estimate s (1 ulp) moved to the neighbour on
+// the other side of x by Tuckerman's test (x <= s (s - ulp): down; x >
+// s (s + ulp): up), whose residuals are exact in that range.
+__device__ __forceinline__ float exact_sqrt_div(float x, float r)
+{
+    const double rd = r, y = __builtin_amdgcn_rcp(rd);
+    const double e = fma(-rd, y, 1.0);
+    const float q = (float)((double)x * fma(y, fma(e, e, e), y));
+    float s = __builtin_amdgcn_sqrtf(q);
+    const float dn = __builtin_bit_cast(float, __builtin_bit_cast(int, s) - 1);
+    const float up = __builtin_bit_cast(float, __builtin_bit_cast(int, s) + 1);
+    const bool lo = fmaf(-dn, s, q) <= 0.0f, hi = fmaf(-up, s, q) > 0.0f;
+    s = lo ? dn : s;
+    s = hi ? up : s;
+    if (!(q >= 0x1p-96f)) s = sqrtf(x / r);
+    return s;
+}
+
+// FP64 has no wider format to round from and divides plainly.  (The compiled
+// sequence without its scaling, the reciprocal shared, behind range tests:
+// 12 % fewer VALU instructions, but 1.06 against 0.97 ms a 256^3 minmod blast
+// step: the tests branch on every face, and the tails ahead of a front leave
+// the range.)
+template <> struct Divisor<double> { double b; };
+__device__ __forceinline__ Divisor<double> make_divisor(double b) { return {b}; }
+__device__ __forceinline__ double exact_div(double a, const Divisor<double> &D) { return a / D.b; }
+__device__ __forceinline__ double exact_rcp(double b) { return 1.0 / b; }
+__device__ __forceinline__ double exact_sqrt_div(double x, double r) { return sqrt(x / r); }
+
 // Whole-wavefront lane shifts (DPP wave_shl:1 / wave_shr:1): lane i receives
 // lane i+1 (shl) or lane i-1 (shr); the lane without a source (63 for shl, 0
 // for shr) keeps `edge` (bound_ctrl off: the destination is not written).
@@ -166,13 +234,16 @@ __device__ __forceinline__ bool wall_ghost(int p, int o, int n, int lo, int hi)
 // calc_primitives (physics.rs:109-141) for one cell.
 // pow2: V is a power of two, so u / V == u * invV exactly.
 template <typename T, bool FAST>
-__device__ __forceinline__ void to_prim(const T u[5], T V, T invV, T gm1, T w[5], bool pow2 = false)
+__device__ __forceinline__ void to_prim(const T u[5], const Divisor<T> &DV, T invV, T gm1, T w[5], bool pow2 = false)
 {
     if constexpr (!FAST) {
-        const T r = pow2 ? u[0] * invV : u[0] / V;
-        const T ux = u[1] / (r * V), uy = u[2] / (r * V), uz = u[3] / (r * V);
+        T r, e;
+        if (pow2) { r = u[0] * invV; e = u[4] * invV; }
+        else { r = exact_div(u[0], DV); e = exact_div(u[4], DV); }
+        const Divisor<T> m = make_divisor(r * DV.b);
+        const T ux = exact_div(u[1], m), uy = exact_div(u[2], m), uz = exact_div(u[3], m);
         w[0] = r; w[1] = ux; w[2] = uy; w[3] = uz;
-        w[4] = ((pow2 ? u[4] * invV : u[4] / V) - T(0.5) * r * (ux * ux + uy * uy + uz * uz)) * gm1;
+        w[4] = (e - T(0.5) * r * (ux * ux + uy * uy + uz * uz)) * gm1;
     } else {
         const T r = u[0] * invV;
         const T im = drcp<T>(u[0]);
@@ -196,11 +267,11 @@ __device__ __forceinline__ T wave_den(const T w[5], T gamma)
 // the sound speed is |x| / sqrt(x U_rho) (one reciprocal square root) and
 // |v| = sqrt(|m|^2) / |U_rho|.
 template <typename T, bool FAST>
-__device__ __forceinline__ T cell_den(const T u[5], T V, T invV, T gm1, T gamma, bool pow2 = false)
+__device__ __forceinline__ T cell_den(const T u[5], const Divisor<T> &DV, T invV, T gm1, T gamma, bool pow2 = false)
 {
     if constexpr (!FAST) {
         T w[5];
-        to_prim<T, false>(u, V, invV, gm1, w, pow2);
+        to_prim<T, false>(u, DV, invV, gm1, w, pow2);
         return wave_den<T, false>(w, gamma);
     } else {
         const T im = drcp<T>(u[0]);
@@ -210,11 +281,37 @@ __device__ __forceinline__ T cell_den(const T u[5], T V, T invV, T gm1, T gamma,
     }
 }
 
+// Exact math: cheap bound for the wave speed of a new state.  The exact
+// evaluation (5-6 divisions, 2 square roots in the reference's order; FP64
+// for the bulk variant) costs ~100 slots per cell, and only the maximum over
+// the grid is used, so a cell whose estimate lies below the largest exact
+// value its wave has found is skipped.  The operations below are good to a
+// few 2^-23; where the internal energy is over 1/8 of the total, the
+// cancellation E - rho v^2 / 2 costs the reference's order and this one at
+// most 2^-19 each, so the estimate is within 2^-18 of the exact value (the
+// floor allows 2^-16); elsewhere, and for anything NaN, negative or out of
+// float's range, it is +inf: evaluate.
+template <typename T>
+__device__ __forceinline__ float den_estimate(const T u[5], float ggm1)
+{
+    const float ur = float(u[0]), mx = float(u[1]), my = float(u[2]), mz = float(u[3]), e = float(u[4]);
+    const float im = __builtin_amdgcn_rcpf(ur);
+    const float ke2 = fmaf(mz, mz * im, fmaf(my, my * im, mx * (mx * im)));   // |m|^2 / U_rho
+    const float ei = fmaf(-0.5f, ke2, e);
+    const float den = __builtin_amdgcn_sqrtf(ei * (ggm1 * im)) + __builtin_amdgcn_sqrtf(ke2 * im);
+    return ei > fmaxf(0.125f * e, 0x1p-80f) && den >= 0.0f ? den : INFINITY;
+}
+
 // Limited slope (extension; the reference's limiters are dead code,
 // physics.f90:205-238): textbook minmod and van Leer.
 template <typename T>
 __device__ __forceinline__ T limited(T a, T b, int lim)
 {
+    if constexpr (sizeof(T) == sizeof(float))
+        if (lim == LIM_MINMOD) {   // of one sign, the smaller magnitude is the median with zero
+            const T m = __builtin_amdgcn_fmed3f(a, b, 0.0f);
+            return a * b > T(0) ? m : T(0);
+        }
     if (!(a * b > T(0))) return T(0);
     if (lim == LIM_MINMOD) return dabs<T>(a) <= dabs<T>(b) ? a : b;
     return T(2) * a * b / (a + b);
@@ -227,31 +324,32 @@ __device__ __forceinline__ T limited(T a, T b, int lim)
 // P = 2 p / (gamma - 1) (so 2 E = rho |v|^2 + P), F is not multiplied by ds,
 // hgm1 = (gamma - 1) / 2 and sK = sqrt(gamma (gamma - 1) / 2).
 template <typename T, bool FAST>
-__device__ __forceinline__ void rusanov(const T l[5], const T r[5], T F[5], T gamma, T gm1, T ds, bool grav, T G,
-                                        T h, T hgm1, T sK)
+__device__ __forceinline__ void rusanov(const T l[5], const T r[5], T F[5], T gamma, const Divisor<T> &dgm1, T ds,
+                                        bool grav, T G, T h, T hgm1, T sK)
 {
     const T rl = l[0], vxl = l[1], vyl = l[2], vzl = l[3], pl = l[4];
     const T rr = r[0], vxr = r[1], vyr = r[2], vzr = r[3], pr = r[4];
     if constexpr (!FAST) {
-        const T en_left = T(0.5) * (rl * (vxl * vxl + vyl * vyl + vzl * vzl)) + (pl / gm1);
-        const T en_right = T(0.5) * (rr * (vxr * vxr + vyr * vyr + vzr * vzr)) + (pr / gm1);
         const T rho_star = (rl + rr) / T(2.0);
         const T mx = (rl * vxl + rr * vxr) / T(2.0);
         const T my = (rl * vyl + rr * vyr) / T(2.0);
         const T mz = (rl * vzl + rr * vzr) / T(2.0);
+        const T c_l = exact_sqrt_div(gamma * pl, rl) + dabs<T>(vxl);
+        const T c_r = exact_sqrt_div(gamma * pr, rr) + dabs<T>(vxr);
+        const T c = dmax<T>(c_l, c_r);
+        const T en_left = T(0.5) * (rl * (vxl * vxl + vyl * vyl + vzl * vzl)) + exact_div(pl, dgm1);
+        const T en_right = T(0.5) * (rr * (vxr * vxr + vyr * vyr + vzr * vzr)) + exact_div(pr, dgm1);
         const T en_star = T(0.5) * (en_left + en_right);
-        const T p_star = gm1 * (en_star - T(0.5) * (mx * mx + my * my + mz * mz) / rho_star);
-        T f1 = (mx * mx / rho_star) + p_star;
-        T f2 = mx * my / rho_star;
-        T f3 = mx * mz / rho_star;
-        T f4 = (en_star + p_star) * (mx / rho_star);
+        const Divisor<T> dr = make_divisor(rho_star);
+        const T p_star = dgm1.b * (en_star - exact_div(T(0.5) * (mx * mx + my * my + mz * mz), dr));
+        T f1 = exact_div(mx * mx, dr) + p_star;
+        T f2 = exact_div(mx * my, dr);
+        T f3 = exact_div(mx * mz, dr);
+        T f4 = (en_star + p_star) * exact_div(mx, dr);
         if (grav) {
             f1 += T(1.0) * rho_star * G * h;
             f4 += T(0.5) * rho_star * (vxl + vxr) * G * h;
         }
-        const T c_l = dsqrt<T>(gamma * pl / rl) + dabs<T>(vxl);
-        const T c_r = dsqrt<T>(gamma * pr / rr) + dabs<T>(vxr);
-        const T c = dmax<T>(c_l, c_r);
         T f0 = mx - T(0.5) * c * (rl - rr);
         f1 -= c * (rl * vxl - rr * vxr) / T(2.0);
         f2 -= c * (rl * vyl - rr * vyr) / T(2.0);
@@ -263,7 +361,7 @@ __device__ __forceinline__ void rusanov(const T l[5], const T r[5], T F[5], T ga
         // caller folds the factor 1/2 and ds into the update).  pl, pr hold
         // P = 2 p / (gamma - 1): the doubled total energies are
         // e2 = m . v + P, and Se2 = 2 Se.
-        (void)gamma; (void)gm1;
+        (void)gamma; (void)dgm1;
         const T mxl = rl * vxl, myl = rl * vyl, mzl = rl * vzl;
         const T mxr = rr * vxr, myr = rr * vyr, mzr = rr * vzr;
         const T e2l = dfma<T>(mzl, vzl, dfma<T>(myl, vyl, dfma<T>(mxl, vxl, pl)));
@@ -311,9 +409,47 @@ __device__ __forceinline__ int rot_field(int axis, int slot)
 template <typename T>
 struct Consts {
     T ds, gamma, gm1, V, invV, two_ds, inv_two_ds, inv_ds, half_ds, half_dt, dtds, G;
+    Divisor<T> dV, dgm1, d2ds, dds;   // exact math: ds^3, gamma - 1, 2 ds, ds as divisors
     T hgm1, sK, irk;   // fast math: (gamma - 1) / 2, sqrt(gamma (gamma - 1) / 2), (gamma - 1) / 2
     bool pow2;   // ds a power of two: divisions by ds, 2 ds, ds^3 as exact products
 };
+
+// Keeps an index computed where it is written (rarely executed branches):
+// hoisted out of the march it would hold a register throughout.
+__device__ __forceinline__ int opaque(int v)
+{
+#ifdef __AMDGCN__
+    asm volatile("" : "+v"(v));
+#endif
+    return v;
+}
+
+// Completes the five values here: otherwise the compiler sinks their last
+// operations past the next branch, and holds all their operands through it.
+template <typename T> __device__ __forceinline__ void complete(T v[5])
+{
+#ifdef __AMDGCN__
+#pragma unroll
+    for (int f = 0; f < 5; ++f) asm volatile("" : "+v"(v[f]));
+#else
+    (void)v;
+#endif
+}
+
+// A wave-uniform value moved to scalar registers (there is no scalar floating
+// point unit, so the compiler keeps uniform arithmetic in VGPRs).
+__device__ __forceinline__ float uniform(float v)
+{ return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v))); }
+__device__ __forceinline__ double uniform(double v)
+{
+    const long long b = __builtin_bit_cast(long long, v);
+    const int lo = __builtin_amdgcn_readfirstlane((int)(b & 0xffffffffLL)), hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
+    return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned int)lo);
+}
+
+// A constant divisor whose reciprocal the host prepared (make_args).
+__device__ __forceinline__ Divisor<float> const_divisor(float b, const DivConst &k) { return {b, k.h, k.l}; }
+__device__ __forceinline__ Divisor<double> const_divisor(double b, const DivConst &) { return {b}; }
 
 // Constants of one step with time step dt.
 template <typename T, bool FAST>
@@ -329,6 +465,10 @@ __device__ __forceinline__ Consts<T> make_consts(const StepArgs &A, T dt)
     C.inv_two_ds = T(1) / C.two_ds;
     C.inv_ds = T(1) / C.ds;
     C.pow2 = A.pow2 != 0;
+    C.dV = const_divisor(C.V, A.dV);
+    C.dgm1 = const_divisor(C.gm1, A.dgm1);
+    C.d2ds = const_divisor(C.two_ds, A.d2ds);
+    C.dds = const_divisor(C.ds, A.dds);
     // fast math: unlimited slopes are central differences (2 ds times the
     // gradient), limited ones one-sided (ds times the gradient)
     const bool one_sided = FAST && A.limiter != LIM_NONE;
@@ -349,8 +489,8 @@ template <typename T> using vec2 = T __attribute__((ext_vector_type(2)));
 
 // LDS layout of the step kernel.
 template <typename T, int TY>
-struct StepLDS {
-    // The primitives ring is cell-major: a cell's 6 words (ring_cell: the
+struct LDSGeom {
+    // The primitives ring W is cell-major: a cell's 6 words (ring_cell: the
     // 5 primitives and, in fast math, its scaled inverse density, the
     // pressure word holding 2 p / (gamma - 1)) are consecutive, read as three
     // pairs; every neighbour of a cell, in all three ring slots, is then
@@ -358,15 +498,40 @@ struct StepLDS {
     static constexpr int NC = (TY + 4) * RZ;  // region cells of one plane
     static constexpr int CS = 6;              // words per cell
     static constexpr int PS = NC * CS;        // one plane
-    alignas(16) T W[3 * PS];  // [plane slot][row][col][ring_cell words]
-    // Ym[.][r]: -y face state of row r (r = 0..TY) until the flux phase, in
-    // which the one thread that reads it replaces it by the flux through
-    // face (r-1, r) (r = 0: the tile's lower y face)
-    T Ym[5][TY + 1][TZ];
-    T Yp[5][TZ];             // +y face state of row -1
-    T Zp[5][TY];             // +z face state of column -1
-    T Zm[5][TY];             // -z face state of column 64
-    T Z0[5][TY];             // -z face state of column 0, then the flux through the tile's lower z face
+};
+// Face states and fluxes beside the ring W:
+// ym row r (0..TY): -y face state of tile row r until the flux phase, in which
+// the one thread that reads it replaces it by the flux through face (r-1, r)
+// (r = 0: the tile's lower y face); yp: +y face state of row -1; zp: +z face
+// state of column -1; zm: -z face state of column 64; z0: -z face state of
+// column 0, then the flux through the tile's lower z face.
+template <typename T, int TY, bool FAST>
+struct StepLDS : LDSGeom<T, TY> {
+    alignas(16) T W[3 * LDSGeom<T, TY>::PS];  // [plane slot][row][col][ring_cell words]
+    T Ym[5][TY + 1][TZ], Yp[5][TZ], Zp[5][TY], Zm[5][TY], Z0[5][TY];
+    __device__ __forceinline__ T &ym(int f, int r, int c) { return Ym[f][r][c]; }
+    __device__ __forceinline__ T &yp(int f, int c) { return Yp[f][c]; }
+    __device__ __forceinline__ T &zp(int f, int r) { return Zp[f][r]; }
+    __device__ __forceinline__ T &zm(int f, int r) { return Zm[f][r]; }
+    __device__ __forceinline__ T &z0(int f, int r) { return Z0[f][r]; }
+};
+// Exact kernels, short of registers: one array with one field stride, so a
+// thread's accesses share address registers, and before the ring, since DS
+// offsets are unsigned 16-bit and an array past 64 KB costs a register per
+// access (FP32, 8 rows: 175 -> 149 VGPRs).  Rows 0..TY are ym, row TY+1 is
+// yp, row TY+2 holds zp, zm and z0.  (The fast kernel measured 2 % slower
+// with it: KHI 512^3 1.826 against 1.787 ms.)
+template <typename T, int TY>
+struct StepLDS<T, TY, false> : LDSGeom<T, TY> {
+    static constexpr int YP = TY + 1, ZB = TY + 2, ZP = 0, ZM = 16, Z0 = 32;
+    static constexpr int FS = (TY + 3) * TZ;  // field stride
+    T E[5][TY + 3][TZ];
+    alignas(16) T W[3 * LDSGeom<T, TY>::PS];
+    __device__ __forceinline__ T &ym(int f, int r, int c) { return E[f][r][c]; }
+    __device__ __forceinline__ T &yp(int f, int c) { return E[f][YP][c]; }
+    __device__ __forceinline__ T &zp(int f, int r) { return E[f][ZB][ZP + r]; }
+    __device__ __forceinline__ T &zm(int f, int r) { return E[f][ZB][ZM + r]; }
+    __device__ __forceinline__ T &z0(int f, int r) { return E[f][ZB][Z0 + r]; }
 };
 
 // The six ring words of a cell from its conserved state u.  Exact math:
@@ -384,7 +549,7 @@ template <typename T, bool FAST>
 __device__ __forceinline__ void ring_cell(const T u[5], const Consts<T> &C, T w[6])
 {
     if constexpr (!FAST) {
-        to_prim<T, false>(u, C.V, C.invV, C.gm1, w, C.pow2);
+        to_prim<T, false>(u, C.dV, C.invV, C.gm1, w, C.pow2);
         w[5] = T(0);
     } else {
         const T im = drcp<T>(u[0]);
@@ -401,16 +566,27 @@ __device__ __forceinline__ void ring_cell(const T u[5], const Consts<T> &C, T w[
 // the limited slope / ds.  Fast math: the same scaled by 2 ds (unlimited) or
 // ds (limited), the factor folded into the constants that consume it.
 template <typename T, bool FAST, int LIM>
-__device__ __forceinline__ T slope(T m, T c, T p, const Consts<T> &C)
+__device__ __forceinline__ T slope_diff(T m, T c, T p)
 {
-    if constexpr (LIM == LIM_NONE) {
-        if constexpr (!FAST) return C.pow2 ? (p - m) * C.inv_two_ds : (p - m) / C.two_ds;
-        else return p - m;
-    } else {
-        if constexpr (!FAST) return C.pow2 ? limited<T>(c - m, p - c, LIM) * C.inv_ds : limited<T>(c - m, p - c, LIM) / C.ds;
-        else if constexpr (LIM == LIM_MINMOD && sizeof(T) == sizeof(float))
-            return __builtin_amdgcn_fmed3f(c - m, p - c, 0.0f);   // minmod(a, b) = median(a, b, 0)
-        else return limited<T>(c - m, p - c, LIM);
+    if constexpr (LIM == LIM_NONE) { (void)c; return p - m; }
+    else if constexpr (FAST && LIM == LIM_MINMOD && sizeof(T) == sizeof(float))
+        return __builtin_amdgcn_fmed3f(c - m, p - c, 0.0f);   // minmod(a, b) = median(a, b, 0)
+    else return limited<T>(c - m, p - c, LIM);
+}
+
+// The division of N slopes by 2 ds or ds (exact math; one branch for all of
+// them: the products with the exact reciprocal when ds is a power of two).
+template <typename T, bool FAST, int LIM, int N>
+__device__ __forceinline__ void scale_slopes(T g[N], const Consts<T> &C)
+{
+    if constexpr (!FAST) {
+        if (C.pow2) {
+#pragma unroll
+            for (int i = 0; i < N; ++i) g[i] = g[i] * (LIM == LIM_NONE ? C.inv_two_ds : C.inv_ds);
+        } else {
+#pragma unroll
+            for (int i = 0; i < N; ++i) g[i] = exact_div(g[i], LIM == LIM_NONE ? C.d2ds : C.dds);
+        }
     }
 }
 
@@ -418,8 +594,9 @@ __device__ __forceinline__ T slope(T m, T c, T p, const Consts<T> &C)
 // mapping does not depend on the plane).  r: flat region index (row*RZ+col)
 // whose slopes and extrapolated state are used; for a wall ghost along y
 // (mask bit 0) or z (bit 1) the normal velocity of xtr flips and the normal
-// slope is evaluated at the ghost's own position ry_wall / rz_wall.
-struct EvalDesc { int r, ry_wall, rz_wall, mask, walls; };   // walls: some lane of the wave has mask != 0
+// slope is evaluated at the ghost's own position, one row or column before r
+// (a lower ghost) or after it (bits 2, 3: an upper one).
+struct EvalDesc { int r, mask, walls; };   // walls: some lane of the wave has a wall ghost
 
 __device__ __forceinline__ EvalDesc make_desc(int py, int pz, int y0, int z0, const StepArgs &A, int ty_max)
 {
@@ -429,9 +606,8 @@ __device__ __forceinline__ EvalDesc make_desc(int py, int pz, int y0, int z0, co
     d.r = (qy + 2) * RZ + (qz + 2);
     d.mask = 0;
     d.walls = 1;
-    d.ry_wall = d.rz_wall = d.r;
-    if (wall_ghost(py, y0, A.n[1], A.bc[2], A.bc[3])) { d.mask |= 1; d.ry_wall = (py + 2) * RZ + (qz + 2); }
-    if (wall_ghost(pz, z0, A.n[2], A.bc[4], A.bc[5])) { d.mask |= 2; d.rz_wall = (qy + 2) * RZ + (pz + 2); }
+    if (wall_ghost(py, y0, A.n[1], A.bc[2], A.bc[3])) d.mask |= py < qy ? 1 : 5;
+    if (wall_ghost(pz, z0, A.n[2], A.bc[4], A.bc[5])) d.mask |= pz < qz ? 2 : 10;
     return d;
 }
 
@@ -472,9 +648,10 @@ __device__ __forceinline__ void hancock(const T w[5], T ir, const T g[15], const
         // physics.rs:251-278, same association
         (void)ir;
         xtr[0] = r - hd * (ux * drx + r * dxx + uy * dry + r * dyy + uz * drz + r * dzz);
-        xtr[1] = ux - hd * (ux * dxx + uy * dxy + uz * dxz + (T(1.0) / r) * dpx);
-        xtr[2] = uy - hd * (ux * dyx + uy * dyy + uz * dyz + (T(1.0) / r) * dpy);
-        xtr[3] = uz - hd * (ux * dzx + uy * dzy + uz * dzz + (T(1.0) / r) * dpz);
+        const T inv_r = exact_rcp(r);
+        xtr[1] = ux - hd * (ux * dxx + uy * dxy + uz * dxz + inv_r * dpx);
+        xtr[2] = uy - hd * (ux * dyx + uy * dyy + uz * dyz + inv_r * dpy);
+        xtr[3] = uz - hd * (ux * dzx + uy * dzy + uz * dzz + inv_r * dpz);
         xtr[4] = p - hd * (C.gamma * p * (dxx + dyy + dzz) + ux * dpx + uy * dpy + uz * dpz);
     } else {
         // hd here is dt / 2 over the slopes' scale (2 ds or ds): slopes are undivided differences
@@ -488,16 +665,18 @@ __device__ __forceinline__ void hancock(const T w[5], T ir, const T g[15], const
 }
 
 template <typename T, int TY, bool FAST, int LIM>
-__device__ __forceinline__ void eval_cell(const StepLDS<T, TY> &L, int sm, int s0, int sp, const EvalDesc &d,
+__device__ __forceinline__ void eval_cell(const StepLDS<T, TY, FAST> &L, int sm, int s0, int sp, const EvalDesc &d,
                                           const Consts<T> &C, T xtr[5], T g[15])
 {
-    constexpr int CS = StepLDS<T, TY>::CS, PS = StepLDS<T, TY>::PS;
-    const T *W0 = L.W + s0 * PS;
-    const T *c0 = W0 + d.r * CS;
+    constexpr int CS = LDSGeom<T, TY>::CS, PS = LDSGeom<T, TY>::PS;
+    // exact math: neighbours are addressed from the cell one row and one column before r
+    constexpr int SH = FAST ? 0 : RZ + 1;
+    const T *b0 = L.W + (d.r - SH) * CS;
+    const T *c0 = b0 + s0 * PS + SH * CS;
     T cc[6], xm[6], xp[6], ym[6], yp[6], zm[6], zp[6];
     ld_cell<T>(c0, cc);
-    ld_prims<T>(L.W + sm * PS + d.r * CS, xm);
-    ld_prims<T>(L.W + sp * PS + d.r * CS, xp);
+    ld_prims<T>(b0 + sm * PS + SH * CS, xm);
+    ld_prims<T>(b0 + sp * PS + SH * CS, xp);
     ld_prims<T>(c0 - RZ * CS, ym);
     ld_prims<T>(c0 + RZ * CS, yp);
     ld_prims<T>(c0 - CS, zm);
@@ -507,27 +686,32 @@ __device__ __forceinline__ void eval_cell(const StepLDS<T, TY> &L, int sm, int s
     for (int f = 0; f < 5; ++f) {
         const T c = cc[f];
         w[f] = c;
-        g[f * 3 + 0] = slope<T, FAST, LIM>(xm[f], c, xp[f], C);
-        g[f * 3 + 1] = slope<T, FAST, LIM>(ym[f], c, yp[f], C);
-        g[f * 3 + 2] = slope<T, FAST, LIM>(zm[f], c, zp[f], C);
+        g[f * 3 + 0] = slope_diff<T, FAST, LIM>(xm[f], c, xp[f]);
+        g[f * 3 + 1] = slope_diff<T, FAST, LIM>(ym[f], c, yp[f]);
+        g[f * 3 + 2] = slope_diff<T, FAST, LIM>(zm[f], c, zp[f]);
     }
+    scale_slopes<T, FAST, LIM, 15>(g, C);
     hancock<T, FAST>(w, cc[5], g, C, xtr);
     if (!d.walls) return;   // wave-uniform: no lane evaluates a wall ghost
     if (d.mask & 1) {   // wall ghost along y: mirrored xtr, slope on the ghost
         xtr[2] = -xtr[2];
+        T q[5];
+        const T *o = L.W + s0 * PS + (opaque(d.r) + (opaque(d.mask) & 4 ? 0 : -2 * RZ)) * CS;   // the ghost's lower neighbour
 #pragma unroll
-        for (int f = 0; f < 5; ++f) {
-            const int o = d.ry_wall * CS + f;
-            g[f * 3 + 1] = slope<T, FAST, LIM>(W0[o - RZ * CS], W0[o], W0[o + RZ * CS], C);
-        }
+        for (int f = 0; f < 5; ++f) q[f] = slope_diff<T, FAST, LIM>(o[f], o[RZ * CS + f], o[2 * RZ * CS + f]);
+        scale_slopes<T, FAST, LIM, 5>(q, C);
+#pragma unroll
+        for (int f = 0; f < 5; ++f) g[f * 3 + 1] = q[f];
     }
     if (d.mask & 2) {
         xtr[3] = -xtr[3];
+        T q[5];
+        const T *o = L.W + s0 * PS + (opaque(d.r) + (opaque(d.mask) & 8 ? 0 : -2)) * CS;
 #pragma unroll
-        for (int f = 0; f < 5; ++f) {
-            const int o = d.rz_wall * CS + f;
-            g[f * 3 + 2] = slope<T, FAST, LIM>(W0[o - CS], W0[o], W0[o + CS], C);
-        }
+        for (int f = 0; f < 5; ++f) q[f] = slope_diff<T, FAST, LIM>(o[f], o[CS + f], o[2 * CS + f]);
+        scale_slopes<T, FAST, LIM, 5>(q, C);
+#pragma unroll
+        for (int f = 0; f < 5; ++f) g[f * 3 + 2] = q[f];
     }
 }
 
@@ -558,7 +742,7 @@ __device__ __forceinline__ void face_flux(const T l[5], const T r[5], int axis, 
     T lr[5], rr[5], F[5];
 #pragma unroll
     for (int s = 0; s < 5; ++s) { lr[s] = l[rot_field(axis, s)]; rr[s] = r[rot_field(axis, s)]; }
-    rusanov<T, FAST>(lr, rr, F, C.gamma, C.gm1, C.ds, grav, C.G, h, C.hgm1, C.sK);
+    rusanov<T, FAST>(lr, rr, F, C.gamma, C.dgm1, C.ds, grav, C.G, h, C.hgm1, C.sK);
 #pragma unroll
     for (int s = 0; s < 5; ++s) out[rot_field(axis, s)] = F[s];
 }
@@ -638,10 +822,10 @@ __device__ __forceinline__ void issue_plane(PlaneLoad<T, TY> &Q, int xg, const L
 }
 
 template <typename T, int TY, bool FAST>
-__device__ __forceinline__ void finish_plane(StepLDS<T, TY> &L, int slot, const PlaneLoad<T, TY> &Q,
+__device__ __forceinline__ void finish_plane(StepLDS<T, TY, FAST> &L, int slot, const PlaneLoad<T, TY> &Q,
                                              const LoadPlan<TY> &P, const Consts<T> &C)
 {
-    constexpr int CS = StepLDS<T, TY>::CS, PS = StepLDS<T, TY>::PS;
+    constexpr int CS = LDSGeom<T, TY>::CS, PS = LDSGeom<T, TY>::PS;
     T *Ws = L.W + slot * PS;
 #pragma unroll
     for (int q = 0; q < LoadPlan<TY>::NS; ++q) {
@@ -663,7 +847,7 @@ __device__ __forceinline__ void finish_plane(StepLDS<T, TY> &L, int slot, const 
 }
 
 template <typename T, int TY, bool FAST>
-__device__ __forceinline__ void load_plane(StepLDS<T, TY> &L, int slot, int xg, const LoadPlan<TY> &P,
+__device__ __forceinline__ void load_plane(StepLDS<T, TY, FAST> &L, int slot, int xg, const LoadPlan<TY> &P,
                                            const StepArgs &A, const Fields<const T> &U, const Consts<T> &C)
 {
     PlaneLoad<T, TY> Q;
@@ -708,7 +892,7 @@ __device__ __forceinline__ void block_partials(double den, int nanf, const doubl
 // (max wave-speed denominator, NaN flag) to partial_out.  Called by the
 // single-grid kernel and by the persistent ensemble kernel.
 template <typename T, int TY, bool FAST, bool BULK, int LIM>
-__device__ __forceinline__ void step_tile(StepLDS<T, TY> &L, double *red, const StepArgs &A,
+__device__ __forceinline__ void step_tile(StepLDS<T, TY, FAST> &L, double *red, const StepArgs &A,
                                           const Fields<const T> &U, const Fields<T> &Vout,
                                           const Scalars *__restrict__ sc, double *__restrict__ partial_out,
                                           int bx, int by, int bz)
@@ -746,6 +930,8 @@ __device__ __forceinline__ void step_tile(StepLDS<T, TY> &L, double *red, const 
     else if (ty == 2 && tz < 2 * TY) halo = make_desc(tz < TY ? tz : tz - TY, tz < TY ? -1 : TZ, y0, z0, A, TY);
     own.walls = __any(own.mask != 0);
     halo.walls = __any(halo.mask != 0);
+    // where this thread's halo face state goes (waves 0-2)
+    T *halo_out = ty == 0 ? &L.yp(0, tz) : (ty == 1 ? &L.ym(0, TY, tz) : (tz < TY ? &L.zp(0, tz) : &L.zm(0, tz - TY)));
     const bool zgrav = A.gravity != 0;
     const T hz = zgrav ? grav_h<T>(zc, nz, C.ds) : T(0);
     // periodic: the reference copies the lower z face from face (n-1, n)
@@ -757,12 +943,15 @@ __device__ __forceinline__ void step_tile(StepLDS<T, TY> &L, double *red, const 
 
     // carried values of the own column
     T xprev[5], gxprev[5];                      // xtr and x-slope of plane t-1
-    T fxlo[5], fyu[5], fyl[5], fzu[5], fzl[5];  // flux parts of plane t-1's cell
+    T fyz[5];                                   // fast math: plane t-1's y/z flux sum minus its lower x face
 #pragma unroll
-    for (int f = 0; f < 5; ++f) { xprev[f] = gxprev[f] = fxlo[f] = fyu[f] = fyl[f] = fzu[f] = fzl[f] = T(0); }
+    for (int f = 0; f < 5; ++f) { xprev[f] = gxprev[f] = fyz[f] = T(0); }
     T maxden = T(0);
     double dmaxden = 0.0;
     int nanf = 0;
+    // exact math: wave speeds below den_floor need no evaluation; a maximum over
+    // den_top raises it (both wave-uniform)
+    float den_floor = -1.0f, den_top = 0.0f;
 
     // the ring holds planes t-1, t, t+1 when plane t's step starts; plane
     // t+2 is loaded during the flux phase of plane t (its slot held t-1,
@@ -774,46 +963,78 @@ __device__ __forceinline__ void step_tile(StepLDS<T, TY> &L, double *red, const 
     load_plane<T, TY, FAST>(L, 1, x0, plan, A, U, C);
     __syncthreads();
 
-    auto plane_step = [&](auto slot, const int t) __attribute__((always_inline)) {
-        constexpr int s0 = decltype(slot)::value, sm = (s0 + 2) % 3, sp = (s0 + 1) % 3;
-        const bool full = t >= x0 && t < xend;
+    // wave speed of a new state, for the next dt
+    auto wave_speed = [&](const T un[5]) __attribute__((always_inline)) {
+        if constexpr (BULK) {
+            T w[5];
+            to_prim<T, FAST>(un, C.dV, C.invV, C.gm1, w, C.pow2);
+            double wd[5];
+            for (int f = 0; f < 5; ++f) wd[f] = (double)w[f];
+            const double den = wave_den<double, false>(wd, (double)C.gamma);
+            nanf |= den != den;
+            dmaxden = fmax(dmaxden, den);   // NaN-ignoring
+        } else {
+            const T den = cell_den<T, FAST>(un, C.dV, C.invV, C.gm1, C.gamma, C.pow2);
+            nanf |= den != den;
+            maxden = dmax<T>(maxden, den);  // NaN-ignoring
+        }
+    };
 
-        // ---- B: halo face states (waves 0-2), then the own cell
+    // ---- B: halo face states (waves 0-2), then the own cell
+    auto eval_phase = [&](auto slot, const bool full, T xtr[5], T g[15], T szm[5]) __attribute__((always_inline)) {
+        constexpr int s0 = decltype(slot)::value, sm = (s0 + 2) % 3, sp = (s0 + 1) % 3;
         if (full && (ty < 2 || (ty == 2 && tz < 2 * TY))) {
-            T hx[5], hg[15], hs[5];
+            // row -1: +y state; row TY: -y; column -1: +z; column 64: -z
+            T hx[5], hg[15];
             eval_cell<T, TY, FAST, LIM>(L, sm, s0, sp, halo, C, hx, hg);
-            if (ty == 0) {                     // row -1: +y state
-                face_state<T, FAST>(hx, hg, 1, true, C, hs);
+            if constexpr (FAST) {
+                T hs[5];
+                if (ty == 0) {
+                    face_state<T, FAST>(hx, hg, 1, true, C, hs);
 #pragma unroll
-                for (int f = 0; f < 5; ++f) L.Yp[f][tz] = hs[f];
-            } else if (ty == 1) {              // row TY: -y state
-                face_state<T, FAST>(hx, hg, 1, false, C, hs);
+                    for (int f = 0; f < 5; ++f) L.yp(f, tz) = hs[f];
+                } else if (ty == 1) {
+                    face_state<T, FAST>(hx, hg, 1, false, C, hs);
 #pragma unroll
-                for (int f = 0; f < 5; ++f) L.Ym[f][TY][tz] = hs[f];
-            } else if (tz < TY) {              // column -1: +z state
-                face_state<T, FAST>(hx, hg, 2, true, C, hs);
+                    for (int f = 0; f < 5; ++f) L.ym(f, TY, tz) = hs[f];
+                } else if (tz < TY) {
+                    face_state<T, FAST>(hx, hg, 2, true, C, hs);
 #pragma unroll
-                for (int f = 0; f < 5; ++f) L.Zp[f][tz] = hs[f];
-            } else {                           // column 64: -z state
-                face_state<T, FAST>(hx, hg, 2, false, C, hs);
+                    for (int f = 0; f < 5; ++f) L.zp(f, tz) = hs[f];
+                } else {
+                    face_state<T, FAST>(hx, hg, 2, false, C, hs);
 #pragma unroll
-                for (int f = 0; f < 5; ++f) L.Zm[f][tz - TY] = hs[f];
+                    for (int f = 0; f < 5; ++f) L.zm(f, tz - TY) = hs[f];
+                }
+            } else {
+                // one store for all four (its address computed once)
+                const bool hplus = ty == 0 || (ty == 2 && tz < TY);
+#pragma unroll
+                for (int f = 0; f < 5; ++f) {
+                    const T q = (ty < 2 ? hg[f * 3 + 1] : hg[f * 3 + 2]) * C.half_ds;
+                    halo_out[f * StepLDS<T, TY, false>::FS] = hplus ? hx[f] + q : hx[f] - q;
+                }
             }
         }
-        T xtr[5], g[15];
         eval_cell<T, TY, FAST, LIM>(L, sm, s0, sp, own, C, xtr, g);
-        T szm[5];
         face_state<T, FAST>(xtr, g, 2, false, C, szm);
         if (full) {
             T sym[5];
             face_state<T, FAST>(xtr, g, 1, false, C, sym);
 #pragma unroll
-            for (int f = 0; f < 5; ++f) L.Ym[f][ty][tz] = sym[f];
+            for (int f = 0; f < 5; ++f) L.ym(f, ty, tz) = sym[f];
             if (tz == 0) {
 #pragma unroll
-                for (int f = 0; f < 5; ++f) L.Z0[f][ty] = szm[f];
+                for (int f = 0; f < 5; ++f) L.z0(f, ty) = szm[f];
             }
         }
+    };
+
+    auto plane_step = [&](auto slot, const int t) __attribute__((always_inline)) {
+        constexpr int sm = (decltype(slot)::value + 2) % 3;
+        const bool full = t >= x0 && t < xend;
+        T xtr[5], g[15], szm[5];
+        eval_phase(slot, full, xtr, g, szm);
         __syncthreads();
 
         // ---- C: fluxes through the own cell's +x (of plane t-1), +y, +z faces;
@@ -850,30 +1071,30 @@ __device__ __forceinline__ void step_tile(StepLDS<T, TY> &L, double *red, const 
             T r[5], l[5];
             face_state<T, FAST>(xtr, g, 1, true, C, r);
 #pragma unroll
-            for (int f = 0; f < 5; ++f) l[f] = L.Ym[f][ty + 1][tz];
+            for (int f = 0; f < 5; ++f) l[f] = L.ym(f, ty + 1, tz);
             face_flux<T, FAST>(l, r, 1, C, false, T(0), fyu_n);
 #pragma unroll
-            for (int f = 0; f < 5; ++f) L.Ym[f][ty + 1][tz] = fyu_n[f];   // read above by this thread only
+            for (int f = 0; f < 5; ++f) L.ym(f, ty + 1, tz) = fyu_n[f];   // read above by this thread only
             face_state<T, FAST>(xtr, g, 2, true, C, r);
 #pragma unroll
-            for (int f = 0; f < 5; ++f) l[f] = from_next_lane<T>(szm[f], L.Zm[f][ty]);
+            for (int f = 0; f < 5; ++f) l[f] = from_next_lane<T>(szm[f], L.zm(f, ty));
             face_flux<T, FAST>(l, r, 2, C, zgrav, hz, fzu_n);
             // the tile's lower y faces (wave 3) and lower z faces (wave 0):
             // waves on the SIMDs that evaluated no halo row in phase B
             if (ty == 3) {
                 T rb[5], lb[5], Fb[5];
 #pragma unroll
-                for (int f = 0; f < 5; ++f) { rb[f] = L.Yp[f][tz]; lb[f] = L.Ym[f][0][tz]; }
+                for (int f = 0; f < 5; ++f) { rb[f] = L.yp(f, tz); lb[f] = L.ym(f, 0, tz); }
                 face_flux<T, FAST>(lb, rb, 1, C, false, T(0), Fb);
 #pragma unroll
-                for (int f = 0; f < 5; ++f) L.Ym[f][0][tz] = Fb[f];
+                for (int f = 0; f < 5; ++f) L.ym(f, 0, tz) = Fb[f];
             } else if (ty == 0 && tz < TY) {
                 T rb[5], lb[5], Fb[5];
 #pragma unroll
-                for (int f = 0; f < 5; ++f) { rb[f] = L.Zp[f][tz]; lb[f] = L.Z0[f][tz]; }
+                for (int f = 0; f < 5; ++f) { rb[f] = L.zp(f, tz); lb[f] = L.z0(f, tz); }
                 face_flux<T, FAST>(lb, rb, 2, C, zgrav, hzb, Fb);
 #pragma unroll
-                for (int f = 0; f < 5; ++f) L.Z0[f][tz] = Fb[f];
+                for (int f = 0; f < 5; ++f) L.z0(f, tz) = Fb[f];
             }
         }
 #pragma unroll
@@ -894,8 +1115,8 @@ __device__ __forceinline__ void step_tile(StepLDS<T, TY> &L, double *red, const 
         if (full) {
 #pragma unroll
             for (int f = 0; f < 5; ++f) {
-                fyl_n[f] = L.Ym[f][ty][tz];
-                fzl_n[f] = from_prev_lane<T>(fzu_n[f], L.Z0[f][ty]);
+                fyl_n[f] = L.ym(f, ty, tz);
+                fzl_n[f] = from_prev_lane<T>(fzu_n[f], L.z0(f, ty));
             }
             if (ylo_out) {                           // boundaries.rs:137-141 on fluxes
 #pragma unroll
@@ -910,56 +1131,178 @@ __device__ __forceinline__ void step_tile(StepLDS<T, TY> &L, double *red, const 
             // outflow at the lower x face: the first cell's lower face copies
             // its upper face (boundaries.rs:107-111 on fluxes)
             const bool xlo_out = xc == 0 && A.bc[0] == BC_OUTFLOW;
-            if constexpr (!FAST) {
-                if (xlo_out) {
-#pragma unroll
-                    for (int f = 0; f < 5; ++f) fxlo[f] = fxu[f];
-                }
-            }
             T un[5];
 #pragma unroll
             for (int f = 0; f < 5; ++f) {
-                const T u = uold[f];
-                T acc;
-                if constexpr (!FAST) acc = ((((fxu[f] - fxlo[f]) + fyu[f]) - fyl[f]) + fzu[f]) - fzl[f];
-                else acc = dfma<T>(xlo_out ? T(0) : T(1), fxu[f], fyu[f]);   // fyu: y/z sum minus the lower x face
-                un[f] = FAST ? dfma<T>(-C.dtds, acc, u) : u - C.dtds * acc;
+                const T acc = dfma<T>(xlo_out ? T(0) : T(1), fxu[f], fyz[f]);
+                un[f] = dfma<T>(-C.dtds, acc, uold[f]);
                 at(Vout.f[f], uidx) = un[f];
             }
-            if constexpr (BULK) {
-                T w[5];
-                to_prim<T, FAST>(un, C.V, C.invV, C.gm1, w, C.pow2);
-                double wd[5];
-                for (int f = 0; f < 5; ++f) wd[f] = (double)w[f];
-                const double den = wave_den<double, false>(wd, (double)C.gamma);
-                nanf |= den != den;
-                dmaxden = fmax(dmaxden, den);   // NaN-ignoring
-            } else {
-                const T den = cell_den<T, FAST>(un, C.V, C.invV, C.gm1, C.gamma, C.pow2);
-                nanf |= den != den;
-                maxden = dmax<T>(maxden, den);  // NaN-ignoring
-            }
+            wave_speed(un);
         }
         if (full) {
             const bool xlo_next = t == 0 && A.bc[0] == BC_OUTFLOW;
 #pragma unroll
             for (int f = 0; f < 5; ++f) {
-                if constexpr (!FAST) {
-                    fxlo[f] = fxu[f];
-                    fyu[f] = fyu_n[f]; fyl[f] = fyl_n[f]; fzu[f] = fzu_n[f]; fzl[f] = fzl_n[f];
-                } else {
-                    const T yz = ((fyu_n[f] - fyl_n[f]) + fzu_n[f]) - fzl_n[f];
-                    fyu[f] = dfma<T>(xlo_next ? T(0) : T(-1), fxu[f], yz);
-                }
+                const T yz = ((fyu_n[f] - fyl_n[f]) + fzu_n[f]) - fzl_n[f];
+                fyz[f] = dfma<T>(xlo_next ? T(0) : T(-1), fxu[f], yz);
             }
         }
     };
+
+    // The exact kernels keep the reference's order of the update,
+    // ((((fx+ - fx-) + fy+) - fy-) + fz+) - fz-, so the four y/z fluxes of a
+    // cell are carried to the next plane, where its upper x face is known: 25
+    // registers.  The x face and the update therefore come first in phase C
+    // and the y and z faces one after the other (the scheduling barriers keep
+    // the compiler from interleaving the three evaluations), which lets the
+    // FP32 kernels fit 128 VGPRs with 9-17 spilled (40 before at 16 rows: 160
+    // bytes of scratch per thread and plane cost more than the arithmetic).
+    // KHI 512^3 FP32: 4.50 -> 3.45 ms a step together with the shared divisions
+    // (1077 -> 855 VALU instructions per 64 cells, 96 % of the issue slots busy);
+    // 256^3 FP32-bulk minmod 0.756 -> 0.490 ms, FP64 minmod 1.03 -> 0.97 ms.
+    T fxlo[5], fyu[5], fyl[5], fzu[5], fzl[5];
+#pragma unroll
+    for (int f = 0; f < 5; ++f) fxlo[f] = fyu[f] = fyl[f] = fzu[f] = fzl[f] = T(0);
+    auto plane_step_exact = [&](auto slot, const int t) __attribute__((always_inline)) {
+        constexpr int sm = (decltype(slot)::value + 2) % 3;
+        const bool full = t >= x0 && t < xend;
+        T xtr[5], g[15], szm[5];
+        eval_phase(slot, full, xtr, g, szm);
+        const int xc = t - 1;
+        const bool upd = xc >= x0 && xc < xend && valid;
+        const uint32_t uidx = (uint32_t)xc * plane_sz + col;
+        __syncthreads();
+        complete(xtr);   // the -z face state is evaluated again below, not kept
+
+        // ---- C: the x face between planes t-1 and t (one evaluation for inner
+        // and boundary planes), then plane t-1's update
+        __builtin_amdgcn_sched_barrier(0);
+        T fxu[5] = {T(0), T(0), T(0), T(0), T(0)}, uold[5];
+        if (t >= x0) {
+            T r[5], l[5];
+            face_state<T, FAST>(xprev, gxprev, 0, true, C, r, 1);
+            face_state<T, FAST>(xtr, g, 0, false, C, l);
+            if ((t == 0 && A.bc[0] == BC_WALL) || (t == nx && A.bc[1] != BC_PERIODIC)) {
+                if (t == 0) {                        // wall: ghost plane -1 mirrors plane 0
+                    T m[5] = {xtr[0], -xtr[1], xtr[2], xtr[3], xtr[4]};
+                    face_state<T, FAST>(m, gxprev, 0, true, C, r, 1);
+                } else if (A.bc[1] == BC_OUTFLOW) {  // ghost nx copies plane nx-1
+                    face_state<T, FAST>(xprev, gxprev, 0, false, C, l, 1);
+                } else {                             // wall: ghost nx mirrors plane nx-1
+                    T m[5] = {xprev[0], -xprev[1], xprev[2], xprev[3], xprev[4]};
+                    face_state<T, FAST>(m, g, 0, false, C, l);
+                }
+            }
+            if (upd) {
+#pragma unroll
+                for (int f = 0; f < 5; ++f) uold[f] = at(U.f[f], uidx);
+            }
+            face_flux<T, FAST>(l, r, 0, C, false, T(0), fxu);
+            complete(fxu);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (upd) {
+            // outflow at the lower x face: the first cell's lower face copies
+            // its upper face (boundaries.rs:107-111 on fluxes)
+            const bool xlo_out = xc == 0 && A.bc[0] == BC_OUTFLOW;
+            T un[5];
+#pragma unroll
+            for (int f = 0; f < 5; ++f) {
+                const T lo = xlo_out ? fxu[f] : fxlo[f];
+                const T acc = ((((fxu[f] - lo) + fyu[f]) - fyl[f]) + fzu[f]) - fzl[f];
+                un[f] = uold[f] - C.dtds * acc;
+                at(Vout.f[f], uidx) = un[f];
+            }
+            if (!(den_estimate<T>(un, float(C.gamma * C.gm1)) < den_floor)) wave_speed(un);
+        }
+        // a lane's maximum has passed what the floor was made of: the wave's
+        // maximum, less the estimate's error, is the new floor (none below
+        // 2^-30, where the estimate loses accuracy)
+        float m = BULK ? (float)dmaxden : (float)maxden;
+        if (__any(m > den_top)) {
+#pragma unroll
+            for (int off = 32; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
+            den_top = uniform(m * (1.0f + 0x1p-16f));
+            den_floor = uniform(m > 0x1p-30f ? m * (1.0f - 0x1p-16f) : -1.0f);
+        }
+#pragma unroll
+        for (int f = 0; f < 5; ++f) { fxlo[f] = fxu[f]; xprev[f] = xtr[f]; gxprev[f] = g[f * 3 + 0]; }
+
+        // the loads of plane t+2, in flight during the y and z faces
+        const bool pre = t + 2 <= xend + 1;
+        PlaneLoad<T, TY> next;
+        if (pre) issue_plane<T, TY>(next, t + 2, plan, A, U);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int f = 0; f < 5; ++f) fyu[f] = fzu[f] = T(0);
+        if (full) {
+            T r[5], l[5];
+            face_state<T, FAST>(xtr, g, 1, true, C, r);
+#pragma unroll
+            for (int f = 0; f < 5; ++f) l[f] = L.ym(f, ty + 1, tz);
+            face_flux<T, FAST>(l, r, 1, C, false, T(0), fyu);
+#pragma unroll
+            for (int f = 0; f < 5; ++f) L.ym(f, ty + 1, tz) = fyu[f];   // read above by this thread only
+            __builtin_amdgcn_sched_barrier(0);
+            face_state<T, FAST>(xtr, g, 2, false, C, l);   // again: five registers fewer until here
+#pragma unroll
+            for (int f = 0; f < 5; ++f) l[f] = from_next_lane<T>(l[f], L.zm(f, ty));
+            face_state<T, FAST>(xtr, g, 2, true, C, r);
+            face_flux<T, FAST>(l, r, 2, C, zgrav, hz, fzu);
+            complete(fzu);
+            __builtin_amdgcn_sched_barrier(0);
+            // the tile's lower y faces (wave 3) and lower z faces (wave 0), one
+            // evaluation for both on rotated states
+            const bool ylow = ty == 3;
+            if (ylow || (ty == 0 && tz < TY)) {
+                T *lo = ylow ? &L.ym(0, 0, tz) : &L.z0(0, tz);
+                const T *hi = ylow ? &L.yp(0, tz) : &L.zp(0, tz);
+                constexpr int FS = StepLDS<T, TY, false>::FS;
+                T rb[5], lb[5], Fb[5];
+#pragma unroll
+                for (int s = 0; s < 5; ++s) {        // slots 1 and 2 (y) or 1, 2, 3 (z) are rotated
+                    rb[s] = ylow ? hi[rot_field(1, s) * FS] : hi[rot_field(2, s) * FS];
+                    lb[s] = ylow ? lo[rot_field(1, s) * FS] : lo[rot_field(2, s) * FS];
+                }
+                rusanov<T, FAST>(lb, rb, Fb, C.gamma, C.dgm1, C.ds, zgrav && !ylow, C.G, hzb, C.hgm1, C.sK);
+#pragma unroll
+                for (int s = 0; s < 5; ++s) {
+                    if (ylow) lo[rot_field(1, s) * FS] = Fb[s];
+                    else lo[rot_field(2, s) * FS] = Fb[s];
+                }
+            }
+        }
+        if (pre) finish_plane<T, TY, FAST>(L, sm, next, plan, C);
+        __syncthreads();
+
+        // ---- D: the lower y/z fluxes of plane t
+        // (of a plane outside the chunk too: unused, but the old values are
+        // then dead through phase C)
+#pragma unroll
+        for (int f = 0; f < 5; ++f) {
+            fyl[f] = L.ym(f, ty, tz);
+            fzl[f] = from_prev_lane<T>(fzu[f], L.z0(f, ty));
+        }
+        if (ylo_out) {                               // boundaries.rs:137-141 on fluxes
+#pragma unroll
+            for (int f = 0; f < 5; ++f) fyl[f] = fyu[f];
+        }
+        if (zlo_tile) {                              // boundaries.rs:167-171 on fluxes
+#pragma unroll
+            for (int f = 0; f < 5; ++f) fzl[f] = zlo_out ? fzu[f] : fzl[f];
+        }
+    };
+    auto advance = [&](auto slot, const int t) __attribute__((always_inline)) {
+        if constexpr (FAST) plane_step(slot, t);
+        else plane_step_exact(slot, t);
+    };
     for (int t = x0 - 1;;) {
-        plane_step(std::integral_constant<int, 0>{}, t);
+        advance(std::integral_constant<int, 0>{}, t);
         if (++t > xend) break;
-        plane_step(std::integral_constant<int, 1>{}, t);
+        advance(std::integral_constant<int, 1>{}, t);
         if (++t > xend) break;
-        plane_step(std::integral_constant<int, 2>{}, t);
+        advance(std::integral_constant<int, 2>{}, t);
         if (++t > xend) break;
     }
 
@@ -968,16 +1311,22 @@ __device__ __forceinline__ void step_tile(StepLDS<T, TY> &L, double *red, const 
     block_partials<NT>(dmaxden, nanf, nosums, red, partial_out, 0, tid);
 }
 
-// Occupancy target: the FP32 fast kernels fit 128 VGPRs (4 waves per SIMD),
-// the FP64 fast kernels 256 (2 waves per SIMD).
-template <typename T, bool FAST> constexpr int waves_per_eu() { return FAST ? (sizeof(T) == 4 ? 4 : 2) : 1; }
+// Occupancy target: the FP32 kernels fit 128 VGPRs (4 waves per SIMD; exact
+// math with 4 rows 168, 3 waves), the FP64 fast kernels 256 (2 waves per SIMD).
+// Exact FP32 at 8 rows: 3.73 ms a KHI 512^3 step with the target, 4.78 without
+// (one workgroup per CU).
+template <typename T, int TY, bool FAST> constexpr int waves_per_eu()
+{
+    if (sizeof(T) == 8) return FAST ? 2 : 1;
+    return FAST || TY > 4 ? 4 : 3;
+}
 
 template <typename T, int TY, bool FAST, bool BULK, int LIM>
-__global__ void __launch_bounds__(TY * TZ) __attribute__((amdgpu_waves_per_eu(waves_per_eu<T, FAST>())))
+__global__ void __launch_bounds__(TY * TZ) __attribute__((amdgpu_waves_per_eu(waves_per_eu<T, TY, FAST>())))
 step_kernel(const StepArgs A, const Fields<const T> U, const Fields<T> Vout, const Scalars *__restrict__ sc,
             double *__restrict__ partials)
 {
-    __shared__ StepLDS<T, TY> L;
+    __shared__ StepLDS<T, TY, FAST> L;
     __shared__ double red[(TY * TZ / 64) * 8];
 #ifdef DG_EMU_POISON
     {   // CPU-emulation builds only: make every unwritten LDS read visible
@@ -1006,7 +1355,7 @@ __global__ void __launch_bounds__(TY * TZ) __attribute__((amdgpu_waves_per_eu(W)
 ens_step_kernel(const EnsInstance *__restrict__ inst, const EnsItem *__restrict__ items, int nitems, int parity,
                 double *__restrict__ partials, int *__restrict__ next)
 {
-    __shared__ StepLDS<T, TY> L;
+    __shared__ StepLDS<T, TY, FAST> L;
     __shared__ double red[(TY * TZ / 64) * 8];
     __shared__ int s_item;
     for (;;) {
@@ -1040,6 +1389,7 @@ reduce_kernel(const StepArgs A, const Fields<const T> U, double *__restrict__ pa
     __shared__ double red[4 * 8];
     const T ds = T(A.ds), gamma = T(A.gamma), gm1 = gamma - T(1.0);
     const T V = ds * ds * ds;
+    const Divisor<T> DV = const_divisor(V, A.dV);
     const size_t n3 = (size_t)A.n[0] * A.n[1] * A.n[2];
     double sums[5] = {0, 0, 0, 0, 0};
     double dmaxden = 0.0;
@@ -1051,13 +1401,13 @@ reduce_kernel(const StepArgs A, const Fields<const T> U, double *__restrict__ pa
         // same math as the step epilogue
         if constexpr (BULK) {
             T w[5];
-            to_prim<T, FAST>(u, V, T(1) / V, gm1, w);
+            to_prim<T, FAST>(u, DV, T(1) / V, gm1, w);
             double wd[5];
             for (int f = 0; f < 5; ++f) wd[f] = (double)w[f];
             const double den = wave_den<double, false>(wd, (double)gamma);
             if (den != den) nanf = 1; else dmaxden = fmax(dmaxden, den);
         } else {
-            const T den = cell_den<T, FAST>(u, V, T(1) / V, gm1, gamma);
+            const T den = cell_den<T, FAST>(u, DV, T(1) / V, gm1, gamma);
             if (den != den) nanf = 1; else maxden = dmax<T>(maxden, den);
         }
     }
@@ -1175,7 +1525,7 @@ cons_to_prim_kernel(const StepArgs A, const Fields<const T> U, const Fields<T> W
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n3; i += (size_t)gridDim.x * blockDim.x) {
         T u[5], w[5];
         for (int f = 0; f < 5; ++f) u[f] = U.f[f][i];
-        to_prim<T, false>(u, V, T(1) / V, gm1, w);
+        to_prim<T, false>(u, const_divisor(V, A.dV), T(1) / V, gm1, w);
         for (int f = 0; f < 5; ++f) W.f[f][i] = w[f];
     }
 }
@@ -1263,7 +1613,7 @@ corr_flag_kernel(const StepArgs A, const Fields<float> U, float *__restrict__ B,
             if (!MASKED) B[q * n3 + i] = up;
             u[q] = up + d[q];
         }
-        to_prim<float, FAST>(u, V, 1.0f / V, gm1, w);
+        to_prim<float, FAST>(u, const_divisor(V, A.dV), 1.0f / V, gm1, w);
         const bool bad = !(w[0] > 0.0f && w[4] > 0.0f);
         if (MASKED) {
             flags[i] = (prev[i] || bad) ? 1 : 0;
@@ -1271,7 +1621,7 @@ corr_flag_kernel(const StepArgs A, const Fields<float> U, float *__restrict__ B,
             flags[i] = bad ? 1 : 0;
             if (bad) atomicAdd(cnt, 1);
             for (int q = 0; q < 5; ++q) U.f[q][i] = u[q];
-            const float den = cell_den<float, FAST>(u, V, 1.0f / V, gm1, gamma);
+            const float den = cell_den<float, FAST>(u, const_divisor(V, A.dV), 1.0f / V, gm1, gamma);
             if (den != den) nanf = 1; else maxden = fmaxf(maxden, den);
         }
     }
@@ -1305,7 +1655,7 @@ corr_apply_kernel(const StepArgs A, const Fields<float> U, const float *__restri
             u[q] = B[q * n3 + i] + d[q];
             U.f[q][i] = u[q];
         }
-        const float den = cell_den<float, FAST>(u, V, 1.0f / V, gm1, gamma);
+        const float den = cell_den<float, FAST>(u, const_divisor(V, A.dV), 1.0f / V, gm1, gamma);
         if (den != den) nanf = 1; else maxden = fmaxf(maxden, den);
     }
     const double nosums[5] = {0, 0, 0, 0, 0};
@@ -1381,7 +1731,8 @@ __device__ __forceinline__ void cell_xtr(const StepArgs &A, const Fields<const T
 #pragma unroll
     for (int f = 0; f < 5; ++f)
 #pragma unroll
-        for (int a = 0; a < 3; ++a) g[f * 3 + a] = slope<T, FAST, LIM>(w[1 + 2 * a][f], w[0][f], w[2 + 2 * a][f], C);
+        for (int a = 0; a < 3; ++a) g[f * 3 + a] = slope_diff<T, FAST, LIM>(w[1 + 2 * a][f], w[0][f], w[2 + 2 * a][f]);
+    scale_slopes<T, FAST, LIM, 15>(g, C);
     hancock<T, FAST>(w[0], w[0][5], g, C, xtr);
 }
 
@@ -1499,7 +1850,7 @@ static void launch_ens_tw(const EnsInstance *inst, const EnsItem *items, int nit
 }
 
 // waves: occupancy target of the FP32 fast kernels (3: up to 168 VGPRs, 4:
-// 128); the other variants are compiled without a target.
+// 128); the other variants take the single-grid kernel's (waves_per_eu).
 template <typename T, int TY, bool FAST, bool BULK>
 static void launch_ens_t(const EnsInstance *inst, const EnsItem *items, int nitems, int grid, int parity,
                          int limiter, double *partials, int *next, int waves, hipStream_t s)
@@ -1508,7 +1859,7 @@ static void launch_ens_t(const EnsInstance *inst, const EnsItem *items, int nite
         if (waves == 3) launch_ens_tw<T, TY, FAST, BULK, 3>(inst, items, nitems, grid, parity, limiter, partials, next, s);
         else launch_ens_tw<T, TY, FAST, BULK, 4>(inst, items, nitems, grid, parity, limiter, partials, next, s);
     } else {
-        launch_ens_tw<T, TY, FAST, BULK, 1>(inst, items, nitems, grid, parity, limiter, partials, next, s);
+        launch_ens_tw<T, TY, FAST, BULK, waves_per_eu<T, TY, FAST>()>(inst, items, nitems, grid, parity, limiter, partials, next, s);
     }
 }
 
@@ -1557,7 +1908,7 @@ static int ens_occ_t(int limiter, int waves)
     if constexpr (FAST && sizeof(T) == 4) {
         return waves == 3 ? ens_occ_tw<T, TY, FAST, BULK, 3>(limiter) : ens_occ_tw<T, TY, FAST, BULK, 4>(limiter);
     } else {
-        return ens_occ_tw<T, TY, FAST, BULK, 1>(limiter);
+        return ens_occ_tw<T, TY, FAST, BULK, waves_per_eu<T, TY, FAST>()>(limiter);
     }
 }
 
@@ -1696,7 +2047,7 @@ int step_lds_bytes(int prec, int tile_y)
 {
     const size_t el = prec == 0 ? sizeof(double) : sizeof(float);
     const size_t ty = (size_t)tile_y;
-    const size_t cells = 3 * 5 * (ty + 4) * RZ + 5 * (ty + 1) * TZ + 2 * 5 * TZ + 5 * ty * TZ + 4 * 5 * ty;
+    const size_t cells = 3 * 6 * (ty + 4) * RZ + 5 * (ty + 3) * TZ;
     return (int)(cells * el + (ty * TZ / 64) * 8 * sizeof(double));
 }
 

@@ -92,6 +92,12 @@ inline float __builtin_amdgcn_sqrtf(float x) { return std::sqrt(x); }
 inline float __builtin_amdgcn_rsqf(float x) { return 1.0f / std::sqrt(x); }
 inline double __builtin_amdgcn_rcp(double x) { return 1.0 / x; }
 inline double __builtin_amdgcn_rsq(double x) { return 1.0 / std::sqrt(x); }
+// v_div_fixup_f32: quotient q of a / b with IEEE zeros, infinities, NaNs and sign
+inline float __builtin_amdgcn_div_fixupf(float q, float b, float a)
+{
+    if (!(std::isfinite(a) && std::isfinite(b)) || a == 0.0f || b == 0.0f) return a / b;
+    return std::signbit(a) != std::signbit(b) ? -std::fabs(q) : std::fabs(q);
+}
 inline float __builtin_amdgcn_fmed3f(float a, float b, float c)   // median of three (ordered inputs)
 {
     return std::max(std::min(a, b), std::min(std::max(a, b), c));
