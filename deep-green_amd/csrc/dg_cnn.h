@@ -39,12 +39,12 @@ enum { CONV_TRAIN = 0, CONV_INFER = 1, CONV_OUT = 2, CONV_BWD = 3, CONV_OUT16 = 
 // (CONV_BWD, full convolution with the flipped weights, times gelu'(Zprev)).
 int conv(int layer, int mode, int B, const int in[3], const void *X, const void *Wp, const float *bias, float *Z,
          void *Xout, float *Y, const float *Zprev, hipStream_t s);
-// Weight gradient of `layer` over a valid convolution with input box `in`:
-// one partial per workgroup (nwg workgroups), then the fixed-order reduction.
-int dw(int layer, int B, const int in[3], const void *X, const void *dZ, float *partials, int nwg, hipStream_t s);
-int dw_tiles(int layer);
-int dw_reduce(int layer, const float *partials, int nwg, float *grad, hipStream_t s);
-int db(const void *dZ, long long ncells, int cpad, int creal, float *partials, int nblk, float *grad, hipStream_t s);
+// Weight and bias gradients of `layer` over a valid convolution with input box
+// `in` (grad: the weights, then the biases): one partial of dw_part_floats
+// floats per workgroup (at most nwg), then the fixed-order reduction.
+constexpr int dw_part_floats = 28 * 32 * 32;
+int dw(int layer, int B, const int in[3], const void *X, const void *dZ, float *partials, int nwg, float *grad,
+       hipStream_t s);
 int pack(int layer, int transpose, const float *W, void *Wp, hipStream_t s);
 int pack_elems(int layer, int transpose);
 int adam(float *w, const float *g, float *m, float *v, int n, float lr, float b1, float b2, float eps, long long t,

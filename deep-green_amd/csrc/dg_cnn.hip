@@ -13,9 +13,9 @@
 //                             read from a ring of input planes in LDS, 16 B
 //                             per lane per k-step (conv_ring_kernel);
 //   weight gradient           D[cout][k] = sum_cells dZ[cell][cout] * X[cell + tap][cin],
-//                             both operands staged channel-major in LDS per
-//                             brick of cells; one partial per workgroup,
-//                             reduced in a fixed order.
+//                             both operands channels-last in LDS, transposed
+//                             by the LDS reads (dw_kernel); one partial per
+//                             workgroup, reduced in a fixed order.
 //
 // MFMA lane layouts (gfx950):
 //   v_mfma_f32_32x32x16_bf16: A lane l holds row l%32, k = 8*(l/32) + i;
@@ -392,163 +392,246 @@ conv_ring_kernel(const RingGeom rg, const bf16 *__restrict__ X, const bf16x8 *__
 }
 
 // ----------------------------------------------------- weight gradient --
-// dW[k][cout] for k = tap*CIN + cin, over the cells of a valid convolution:
-// sum_cells dZ[cell][cout] * X[cell + tap][cin].  Bricks of 2 x 4 x 32 output
-// cells; LDS holds the input brick (4 x 6 x 34) and the dZ brick channel-major.
-constexpr int DW_BX = 2, DW_BY = 4, DW_BZ = 32;
-constexpr int DW_IX = DW_BX + 2, DW_IY = DW_BY + 2, DW_IZ = DW_BZ + 2;
+// dW[tap][cin][cout] = sum over the cells of a valid convolution of
+// dZ[cell][cout] * X[cell + tap][cin], and db[cout] = sum of dZ, as an MFMA
+// GEMM with K = cells: A = dZ^T (32 output channels), B = X at one tap (32
+// input channels of a tile; with CIN 8 four taps of 8) or ones (the tap after
+// the last, whose columns are the bias gradient).
+//
+// Both operands need 8 consecutive cells of one channel per lane, but the
+// activations are channels-last.  They stay so in LDS, and
+// ds_read_b64_tr_b16 transposes on the way to the registers: 16 lanes read 4
+// cells x 16 channels, lane i receives channel i of the 4 cells, and since
+// every cell has its own address a tap is an offset like any other.
+// A workgroup owns a rectangle of ry x rz outputs in (y, z) and marches along
+// x over a chunk of planes: a ring of 4 input planes (rows of 48 cells, so
+// that taps are constant offsets) and 2 dZ planes, the next ones loaded to
+// registers before a plane's MFMAs and stored after them (one barrier per
+// plane).  The 28 column tiles (7 with CIN 8) are 7 per wave, held in the
+// accumulators to the end: TG waves split the tiles and KG split the cells
+// (16 per MFMA); the KG sums are added in LDS in a fixed order and each
+// workgroup writes one partial (deterministic).
+// Bound by LDS: 8 KB of transposed reads per 7 MFMAs and wave, and the
+// staging.  A training batch of 8 crops of 32^3: layers 1-3 in 22, 39 and 35
+// us; before, staged channel-major with 2-byte writes and gathered with eight
+// 2-byte reads per MFMA, 113, 220 and 200 us, and 41 us for each layer's
+// separate bias sums (the Adam step 1.08 -> 0.50 ms).
+constexpr int DW_WAVES = 8;
+constexpr int DW_ROWP = 48, DW_RMAX = 9;                     // LDS rows of 48 cells, at most 9
+constexpr int DW_POS = (DW_RMAX - 2) * (DW_ROWP - 2);        // outputs per rectangle and plane
+constexpr int DW_ZCELLS = (DW_POS + 15) / 16 * 16;
+
+struct DwGeom {
+    ConvGeom g;
+    int ry, rz, magic;   // rectangle; cell / rz == cell * magic >> 16
+    int ny, nz;          // rectangles along y, z
+    int cx, nxc;         // output planes per work item, chunks along x
+    long long items;
+};
+
+template <int CIN, int COUT> struct DwCfg {
+    static constexpr int XB = CIN * 2, ZB = COUT * 2;        // bytes per cell
+    static constexpr int XSLOT = DW_RMAX * DW_ROWP * XB, ZSLOT = DW_ZCELLS * ZB;
+    static constexpr int NTILES = 28 * CIN / 32;
+    static constexpr int TPW = 7, TG = NTILES / TPW, KG = DW_WAVES / TG;
+    static constexpr int STAGE = 4 * XSLOT + 2 * ZSLOT, RED = DW_WAVES / 2 * TPW * 64 * 16 * 4;
+    static constexpr int LDS = STAGE > RED ? STAGE : RED;
+    static constexpr int XPER = (DW_RMAX * DW_ROWP * (CIN / 8) + 64 * DW_WAVES - 1) / (64 * DW_WAVES);
+    static constexpr int ZPER = (DW_POS * (COUT / 8) + 64 * DW_WAVES - 1) / (64 * DW_WAVES);
+};
+
+#ifdef __HIP__
+typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
+#else
+typedef bf16x4 lds_bf16x4;
+#endif
+// 8 cells (rows a and b of this lane's two transposed reads) of one channel
+__device__ __forceinline__ bf16x8 read_tr(char *a, char *b)
+{
+    const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4 *)a);
+    const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4 *)b);
+    return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+}
 
 template <int CIN, int COUT>
-__global__ void __launch_bounds__(512)
-dw_kernel(const ConvGeom g, const bf16 *__restrict__ X, const bf16 *__restrict__ dZ, float *__restrict__ partials)
+__global__ void __launch_bounds__(64 * DW_WAVES) __attribute__((amdgpu_waves_per_eu(2, 2)))
+dw_kernel(const DwGeom dg, const bf16 *__restrict__ X, const bf16 *__restrict__ dZ, float *__restrict__ partials)
 {
-    constexpr int NCOL = 27 * CIN;
-    constexpr int NTILES = (NCOL + 31) / 32;
-    constexpr int TPW = (NTILES + 7) / 8;
-    __shared__ __attribute__((aligned(16))) bf16 xs[CIN][DW_IX][DW_IY][DW_IZ];
-    __shared__ __attribute__((aligned(16))) bf16 zs[32][DW_BX][DW_BY][DW_BZ];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, h = lane / 32;
-    const int nbx = (g.out[0] + DW_BX - 1) / DW_BX, nby = (g.out[1] + DW_BY - 1) / DW_BY,
-              nbz = (g.out[2] + DW_BZ - 1) / DW_BZ;
-    const long long nbricks = (long long)g.B * nbx * nby * nbz;
+    typedef DwCfg<CIN, COUT> C;
+    constexpr int TPW = C::TPW, NC = CIN / 8, NZ = COUT / 8, NT = 64 * DW_WAVES;
+    __shared__ __attribute__((aligned(16))) char lds[C::LDS];
+    char *const xr = lds, *const zr = lds + 4 * C::XSLOT;
+    const ConvGeom &g = dg.g;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tg = wave % C::TG, kg = wave / C::TG;
+    // transposed reads: this lane's address is row kr (and kr + 4) of the 16
+    // cells, 4 channels from ch; its result is column 16 * half + j
+    const int half = (lane >> 4) & 1, j = lane & 15;
+    const int kr = 8 * (lane >> 5) + (j >> 2);
+    const int npos = dg.ry * dg.rz, nkb = (npos + 15) / 16;
 
-    // columns of this wave's tiles
-    int ctap[TPW], ccin[TPW];
-    bool cok[TPW];
-#pragma unroll
-    for (int q = 0; q < TPW; ++q) {
-        const int n = (wave + 8 * q) * 32 + (lane % 32);
-        cok[q] = (wave + 8 * q) < NTILES && n < NCOL;
-        ctap[q] = cok[q] ? n / CIN : 0;
-        ccin[q] = cok[q] ? n % CIN : 0;
-    }
+    // the dZ slots past npos stay zero
+    for (int e = tid * 16; e < 2 * C::ZSLOT; e += NT * 16) *reinterpret_cast<u32x4 *>(zr + e) = u32x4{0, 0, 0, 0};
+
     f32x16 acc[TPW];
 #pragma unroll
-    for (int q = 0; q < TPW; ++q)
+    for (int t = 0; t < TPW; ++t)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) acc[q][i] = 0.0f;
+        for (int i = 0; i < 16; ++i) acc[t][i] = 0.0f;
 
-    for (long long br = blockIdx.x; br < nbricks; br += gridDim.x) {
-        long long r = br;
-        const int bz = (int)(r % nbz); r /= nbz;
-        const int by = (int)(r % nby); r /= nby;
-        const int bx = (int)(r % nbx); r /= nbx;
-        const int b = (int)r;
-        const int x0 = bx * DW_BX, y0 = by * DW_BY, z0 = bz * DW_BZ;
-        // stage X (input brick) and dZ (output brick), channel-major, zeros outside
-        constexpr int XCH = CIN / 8;
-        for (int e = tid; e < DW_IX * DW_IY * DW_IZ * XCH; e += 512) {
-            const int c8 = e % XCH, cell = e / XCH;
-            const int iz = cell % DW_IZ, iy = (cell / DW_IZ) % DW_IY, ix = cell / (DW_IZ * DW_IY);
-            const int gx = x0 + ix, gy = y0 + iy, gz = z0 + iz;
-            bf16x8 v = zero8();
-            if (gx < g.in[0] && gy < g.in[1] && gz < g.in[2])
-                v = *reinterpret_cast<const bf16x8 *>(
-                    X + ((((long long)b * g.in[0] + gx) * g.in[1] + gy) * g.in[2] + gz) * CIN + c8 * 8);
+    u32x4 xv[C::XPER], zv[C::ZPER];
+    int b = 0, y0 = 0, z0 = 0;
+    auto load_x = [&](int xi) {
+        const long long pb = ((long long)b * g.in[0] + xi) * g.in[1];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) xs[c8 * 8 + i][ix][iy][iz] = v[i];
+        for (int k = 0; k < C::XPER; ++k) {
+            const int idx = k * NT + tid, cell = idx / NC, q = idx % NC;
+            const int yi = y0 + cell / DW_ROWP, zi = z0 + cell % DW_ROWP;
+            const bool in = cell / DW_ROWP < dg.ry + 2 && cell % DW_ROWP < dg.rz + 2 && xi < g.in[0] && yi < g.in[1] &&
+                            zi < g.in[2];
+            xv[k] = in ? *reinterpret_cast<const u32x4 *>(X + ((pb + yi) * g.in[2] + zi) * CIN + q * 8)
+                       : u32x4{0, 0, 0, 0};
         }
-        constexpr int ZCH = COUT / 8;
-        for (int e = tid; e < DW_BX * DW_BY * DW_BZ * 4; e += 512) {
-            const int c8 = e % 4, cell = e / 4;
-            const int iz = cell % DW_BZ, iy = (cell / DW_BZ) % DW_BY, ix = cell / (DW_BZ * DW_BY);
-            const int gx = x0 + ix, gy = y0 + iy, gz = z0 + iz;
-            bf16x8 v = zero8();
-            if (c8 < ZCH && gx < g.out[0] && gy < g.out[1] && gz < g.out[2])
-                v = *reinterpret_cast<const bf16x8 *>(
-                    dZ + ((((long long)b * g.out[0] + gx) * g.out[1] + gy) * g.out[2] + gz) * COUT + c8 * 8);
+    };
+    auto store_x = [&](int xi) {
+        char *slot = xr + (xi & 3) * C::XSLOT;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) zs[c8 * 8 + i][ix][iy][iz] = v[i];
+        for (int k = 0; k < C::XPER; ++k) {
+            const int idx = k * NT + tid, cell = idx / NC, q = idx % NC;
+            if (cell / DW_ROWP < dg.ry + 2 && cell % DW_ROWP < dg.rz + 2)
+                *reinterpret_cast<u32x4 *>(slot + cell * C::XB + q * 16) = xv[k];
         }
+    };
+    auto load_z = [&](int x) {
+        const long long pb = ((long long)b * g.out[0] + x) * g.out[1];
+#pragma unroll
+        for (int k = 0; k < C::ZPER; ++k) {
+            const int idx = k * NT + tid, cell = idx / NZ, q = idx % NZ;
+            const int r = cell * dg.magic >> 16, yi = y0 + r, zi = z0 + cell - r * dg.rz;
+            const bool in = cell < npos && yi < g.out[1] && zi < g.out[2];
+            zv[k] = in ? *reinterpret_cast<const u32x4 *>(dZ + ((pb + yi) * g.out[2] + zi) * COUT + q * 8)
+                       : u32x4{0, 0, 0, 0};
+        }
+    };
+    auto store_z = [&](int x) {
+        char *slot = zr + (x & 1) * C::ZSLOT;
+#pragma unroll
+        for (int k = 0; k < C::ZPER; ++k) {
+            const int idx = k * NT + tid;
+            if (idx / NZ < npos) *reinterpret_cast<u32x4 *>(slot + idx * 16) = zv[k];
+        }
+    };
+
+    for (long long item = blockIdx.x; item < dg.items; item += gridDim.x) {
+        long long r = item;
+        z0 = (int)(r % dg.nz) * dg.rz; r /= dg.nz;
+        y0 = (int)(r % dg.ny) * dg.ry; r /= dg.ny;
+        const int xs = (int)(r % dg.nxc) * dg.cx, xe = min(xs + dg.cx, g.out[0]);
+        b = (int)(r / dg.nxc);
+        __syncthreads();   // the zeroed dZ slots
+#pragma unroll
+        for (int k = 0; k < 3; ++k) { load_x(xs + k); store_x(xs + k); }
+        load_z(xs);
+        store_z(xs);
         __syncthreads();
-        for (int x = 0; x < DW_BX; ++x)
-            for (int y = 0; y < DW_BY; ++y)
-                for (int zk = 0; zk < DW_BZ; zk += 16) {
-                    // A = dZ^T: row cout = lane%32, k = cells z = zk + 8h + i
-                    const bf16x8 a = *reinterpret_cast<const bf16x8 *>(&zs[lane % 32][x][y][zk + 8 * h]);
+        for (int x = xs; x < xe; ++x) {
+            const bool more = x + 1 < xe;
+            if (more) { load_x(x + 3); load_z(x + 1); }
+            // this lane's part of the tiles' input addresses
+            char *tb[TPW];
 #pragma unroll
-                    for (int q = 0; q < TPW; ++q) {
-                        const int tap = ctap[q], cin = ccin[q];
-                        const int dx = tap / 9, dy = (tap / 3) % 3, dz = tap % 3;
-                        bf16x8 bv;
+            for (int t = 0; t < TPW; ++t) {
+                int tap, ch;
+                if (CIN == 32) { tap = tg * TPW + t; ch = 16 * half + 4 * (j & 3); }
+                else { tap = 4 * t + 2 * half + ((j & 3) >> 1); ch = 4 * (j & 1); }
+                if (tap == 27) tap = 0;
+                const int dx = tap / 9, dy = tap / 3 % 3, dz = tap % 3;
+                tb[t] = xr + ((x + dx) & 3) * C::XSLOT + (dy * DW_ROWP + dz) * C::XB + ch * 2;
+            }
+            char *zb = zr + (x & 1) * C::ZSLOT + (COUT == 32 ? 16 * half : 0) * 2 + 8 * (j & 3);
+            for (int kb = kg; kb < nkb; kb += C::KG) {
+                const int i0 = kb * 16 + kr, i1 = i0 + 4;
+                bf16x8 a = read_tr(zb + i0 * C::ZB, zb + i1 * C::ZB);
+                if (COUT == 16 && half) a = zero8();
+                const int c0 = i0 < npos ? i0 : npos - 1, c1 = i1 < npos ? i1 : npos - 1;
+                const int r0 = c0 * dg.magic >> 16, r1 = c1 * dg.magic >> 16;
+                const int o0 = (r0 * (DW_ROWP - dg.rz) + c0) * C::XB, o1 = (r1 * (DW_ROWP - dg.rz) + c1) * C::XB;
 #pragma unroll
-                        for (int i = 0; i < 8; ++i) bv[i] = xs[cin][x + dx][y + dy][zk + 8 * h + i + dz];
-                        if (!cok[q]) bv = zero8();
-                        acc[q] = Mfma<32>::op(a, bv, acc[q]);
+                for (int t = 0; t < TPW; ++t) {
+                    bf16x8 bv = read_tr(tb[t] + o0, tb[t] + o1);
+                    if (t == TPW - 1) {   // the bias columns
+                        const bool one = CIN == 32 ? tg == C::TG - 1 : 2 * half + (j >> 3) == 3;
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) bv[i] = one ? (bf16)1.0f : bv[i];
                     }
+                    acc[t] = Mfma<32>::op(a, bv, acc[t]);
                 }
-        __syncthreads();
+            }
+            if (more) { store_x(x + 3); store_z(x + 1); }
+            __syncthreads();
+        }
     }
-    // partial of this workgroup: [NTILES*32 columns][32 couts]
-    float *P = partials + (size_t)blockIdx.x * NTILES * 32 * 32;
+
+    // add the KG sums of every tile (halves, in a fixed order), then one
+    // partial per workgroup: [column][32 couts]
+    float *red = reinterpret_cast<float *>(lds);
 #pragma unroll
-    for (int q = 0; q < TPW; ++q) {
-        const int T = wave + 8 * q;
-        if (T >= NTILES) continue;
-        const int n = T * 32 + lane % 32;
+    for (int s = C::KG / 2; s >= 1; s >>= 1) {
+        __syncthreads();
+        if (kg >= s && kg < 2 * s) {
+            float *o = red + ((kg - s) * C::TG + tg) * TPW * 1024 + lane * 4;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) P[(size_t)n * 32 + Mfma<32>::row(i, lane)] = acc[q][i];
+            for (int t = 0; t < TPW; ++t)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    *reinterpret_cast<f32x4 *>(o + t * 1024 + q * 256) =
+                        f32x4{acc[t][4 * q], acc[t][4 * q + 1], acc[t][4 * q + 2], acc[t][4 * q + 3]};
+        }
+        __syncthreads();
+        if (kg < s) {
+            const float *o = red + (kg * C::TG + tg) * TPW * 1024 + lane * 4;
+#pragma unroll
+            for (int t = 0; t < TPW; ++t)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const f32x4 v = *reinterpret_cast<const f32x4 *>(o + t * 1024 + q * 256);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) acc[t][4 * q + i] += v[i];
+                }
+        }
+    }
+    if (kg == 0) {
+        float *P = partials + (size_t)blockIdx.x * C::NTILES * 1024;
+#pragma unroll
+        for (int t = 0; t < TPW; ++t)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                *reinterpret_cast<f32x4 *>(P + ((tg * TPW + t) * 32 + lane % 32) * 32 + Mfma<32>::row(4 * q, lane)) =
+                    f32x4{acc[t][4 * q], acc[t][4 * q + 1], acc[t][4 * q + 2], acc[t][4 * q + 3]};
     }
 }
 
-// grad[tap][cin_real][cout_real] = sum over workgroups of the partials:
-// one block per (tap, cin); 8 groups of 32 lanes (one per output channel)
-// each sum every 8th workgroup in order, then the 8 group sums are added in
-// order (a fixed order: deterministic).
+// grad[tap][cin_real][cout_real] and, after it, the bias gradient: the sum
+// over workgroups of the partials.  One block per (tap, cin), the last one for
+// the bias column; 8 groups of 32 lanes (one per output channel) each sum
+// every 8th workgroup in order, then the 8 group sums are added in order (a
+// fixed order: deterministic).
 __global__ void __launch_bounds__(256)
 dw_reduce_kernel(const float *__restrict__ partials, int nwg, int cin_pad, int cin_real, int cout_real,
                  float *__restrict__ grad)
 {
     __shared__ double red[8][32];
-    const int ncol = 27 * cin_pad;
-    const int ntiles = (ncol + 31) / 32;
-    const int tap = blockIdx.x / cin_real, ci = blockIdx.x % cin_real;
+    const int tap = blockIdx.x / cin_real, ci = blockIdx.x % cin_real;   // tap 27: bias
     const int n = tap * cin_pad + ci;
     const int co = threadIdx.x & 31, grp = threadIdx.x >> 5;
     double s = 0.0;
-    for (int w = grp; w < nwg; w += 8) s += (double)partials[((size_t)w * ntiles * 32 + n) * 32 + co];
+    for (int w = grp; w < nwg; w += 8) s += (double)partials[((size_t)w * 28 * cin_pad + n) * 32 + co];
     red[grp][co] = s;
     __syncthreads();
     if (grp == 0 && co < cout_real) {
         double t = 0.0;
         for (int q = 0; q < 8; ++q) t += red[q][co];
         grad[(size_t)blockIdx.x * cout_real + co] = (float)t;
-    }
-}
-
-// bias gradient: db[c] = sum over cells of dZ[cell][c] (partials per block)
-__global__ void __launch_bounds__(256)
-db_kernel(const bf16 *__restrict__ dZ, long long ncells, int cpad, float *__restrict__ partials)
-{
-    __shared__ float red[256];
-    const int c = threadIdx.x % 32, r = threadIdx.x / 32;
-    float s = 0.0f;
-    if (c < cpad)
-        for (long long m = (long long)blockIdx.x * 8 + r; m < ncells; m += (long long)gridDim.x * 8)
-            s += (float)dZ[m * cpad + c];
-    red[threadIdx.x] = s;
-    __syncthreads();
-    if (r == 0) {
-        for (int q = 1; q < 8; ++q) s += red[q * 32 + c];
-        partials[blockIdx.x * 32 + c] = s;
-    }
-}
-
-// grad[c] = sum over blocks of the partials: 8 groups of 32 channels each sum
-// every 8th block in order, then the group sums are added in order.
-__global__ void __launch_bounds__(256)
-db_reduce_kernel(const float *__restrict__ partials, int nblk, int creal, float *__restrict__ grad)
-{
-    __shared__ double red[8][32];
-    const int c = threadIdx.x & 31, grp = threadIdx.x >> 5;
-    double s = 0.0;
-    for (int b = grp; b < nblk; b += 8) s += (double)partials[b * 32 + c];
-    red[grp][c] = s;
-    __syncthreads();
-    if (grp == 0 && c < creal) {
-        double t = 0.0;
-        for (int q = 0; q < 8; ++q) t += red[q][c];
-        grad[c] = (float)t;
     }
 }
 
@@ -828,35 +911,54 @@ int conv(int layer, int mode, int B, const int in[3], const void *X, const void 
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
-int dw_tiles(int layer)
+// Rectangles of at most 7 x 46 outputs: rz balanced over the extent, ry the
+// one that leaves the fewest 16-cell blocks (rounded up to the waves that
+// split them); x chunks so that the work items fill nwg workgroups once.
+static DwGeom dw_geom(const ConvGeom &g, int kgroups, int nwg)
 {
-    const int cin = layer == 1 ? 8 : 32;
-    return (27 * cin + 31) / 32;
+    DwGeom d;
+    d.g = g;
+    d.nz = (g.out[2] + DW_ROWP - 3) / (DW_ROWP - 2);
+    d.rz = (g.out[2] + d.nz - 1) / d.nz;
+    d.magic = (65536 + d.rz - 1) / d.rz;
+    long long best = -1;
+    d.ry = 1;
+    for (int ry = 1; ry <= DW_RMAX - 2 && ry <= g.out[1]; ++ry) {
+        const long long rows = (g.out[1] + ry - 1) / ry, blocks = (ry * d.rz + 16 * kgroups - 1) / (16 * kgroups);
+        const long long cost = rows * (4 * blocks + ry + 4);   // MFMAs, staging and a barrier per plane
+        if (best < 0 || cost <= best) { best = cost; d.ry = ry; }
+    }
+    d.ny = (g.out[1] + d.ry - 1) / d.ry;
+    const long long cols = (long long)g.B * d.ny * d.nz;
+    long long nxc = nwg / cols;
+    if (nxc > g.out[0]) nxc = g.out[0];
+    if (nxc < 1) nxc = 1;
+    d.cx = (int)((g.out[0] + nxc - 1) / nxc);
+    d.nxc = (g.out[0] + d.cx - 1) / d.cx;
+    d.items = cols * d.nxc;
+    return d;
 }
 
-int dw(int layer, int B, const int in[3], const void *X, const void *dZ, float *partials, int nwg, hipStream_t s)
+template <int CIN, int COUT>
+static int launch_dw(const ConvGeom &g, const void *X, const void *dZ, float *partials, int nwg, hipStream_t s)
+{
+    const DwGeom d = dw_geom(g, DwCfg<CIN, COUT>::KG, nwg);
+    const int blocks = (int)(d.items < nwg ? d.items : nwg);
+    hipLaunchKernelGGL((dw_kernel<CIN, COUT>), dim3(blocks), dim3(64 * DW_WAVES), 0, s, d, static_cast<const bf16 *>(X),
+                       static_cast<const bf16 *>(dZ), partials);
+    return blocks;
+}
+
+int dw(int layer, int B, const int in[3], const void *X, const void *dZ, float *partials, int nwg, float *grad,
+       hipStream_t s)
 {
     const ConvGeom g = geom(B, in, 0);
-    const bf16 *x = static_cast<const bf16 *>(X);
-    const bf16 *z = static_cast<const bf16 *>(dZ);
-    if (layer == 1) hipLaunchKernelGGL((dw_kernel<8, 32>), dim3(nwg), dim3(512), 0, s, g, x, z, partials);
-    else if (layer == 2) hipLaunchKernelGGL((dw_kernel<32, 32>), dim3(nwg), dim3(512), 0, s, g, x, z, partials);
-    else hipLaunchKernelGGL((dw_kernel<32, 16>), dim3(nwg), dim3(512), 0, s, g, x, z, partials);
-    return hipGetLastError() == hipSuccess ? 0 : -2;
-}
-
-int dw_reduce(int layer, const float *partials, int nwg, float *grad, hipStream_t s)
-{
     const int cin_pad = layer == 1 ? 8 : 32, cin_real = layer == 1 ? 5 : 32, cout_real = layer == 3 ? 15 : 32;
-    hipLaunchKernelGGL(dw_reduce_kernel, dim3(27 * cin_real), dim3(256), 0, s, partials, nwg, cin_pad, cin_real,
+    const int blocks = layer == 1 ? launch_dw<8, 32>(g, X, dZ, partials, nwg, s)
+                       : layer == 2 ? launch_dw<32, 32>(g, X, dZ, partials, nwg, s)
+                                    : launch_dw<32, 16>(g, X, dZ, partials, nwg, s);
+    hipLaunchKernelGGL(dw_reduce_kernel, dim3(27 * cin_real + 1), dim3(256), 0, s, partials, blocks, cin_pad, cin_real,
                        cout_real, grad);
-    return hipGetLastError() == hipSuccess ? 0 : -2;
-}
-
-int db(const void *dZ, long long ncells, int cpad, int creal, float *partials, int nblk, float *grad, hipStream_t s)
-{
-    hipLaunchKernelGGL(db_kernel, dim3(nblk), dim3(256), 0, s, static_cast<const bf16 *>(dZ), ncells, cpad, partials);
-    hipLaunchKernelGGL(db_reduce_kernel, dim3(1), dim3(256), 0, s, partials, nblk, creal, grad);
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 

@@ -40,7 +40,6 @@ const int64_t kW1 = 0, kB1 = kW1 + 27 * 5 * 32, kW2 = kB1 + 32, kB2 = kW2 + 27 *
               kB3 = kW3 + 27 * 32 * 15, kNParams = kB3 + 15;
 const int64_t kWoff[3] = {kW1, kW2, kW3}, kBoff[3] = {kB1, kB2, kB3};
 const int kDwGroups = 256;     // workgroups of the weight-gradient kernels
-const int kDbBlocks = 256;     // blocks of the bias-gradient kernels
 const int kLossBlocks = 256;
 const int kGraphSteps = 16;
 
@@ -73,7 +72,7 @@ struct dg_cnn {
     size_t tmp_cells = 0;
     // workspaces
     Buf ws[16];
-    float *dw_part = nullptr, *db_part = nullptr;
+    float *dw_part = nullptr;
     double *loss_part = nullptr;
     // inference tables (per buffer parity of the coarse context)
     const float **d_ptrs = nullptr;       // [2][5]
@@ -173,21 +172,15 @@ int backward(dg_cnn *m, int B, const int in[3])
     if (!dZ2 || !dZ1) return mfail(m, DG_ERR_ALLOC, "workspace");
     void *dG = m->ws[WS_DG].p;
     // layer 3
-    MCHK(m, dg::cnn::dw(3, B, d2, m->ws[WS_X2].p, dG, m->dw_part, kDwGroups, m->stream), "dw3");
-    MCHK(m, dg::cnn::dw_reduce(3, m->dw_part, kDwGroups, m->grads + kW3, m->stream), "dw3 reduce");
-    MCHK(m, dg::cnn::db(dG, (long long)c3, 16, 15, m->db_part, kDbBlocks, m->grads + kB3, m->stream), "db3");
+    MCHK(m, dg::cnn::dw(3, B, d2, m->ws[WS_X2].p, dG, m->dw_part, kDwGroups, m->grads + kW3, m->stream), "dw3");
     MCHK(m, dg::cnn::conv(3, dg::cnn::CONV_BWD, B, d3, dG, m->Wt[2], nullptr, nullptr, dZ2, nullptr,
                           (const float *)m->ws[WS_Z2].p, m->stream), "conv3 bwd");
     // layer 2
-    MCHK(m, dg::cnn::dw(2, B, d1, m->ws[WS_X1].p, dZ2, m->dw_part, kDwGroups, m->stream), "dw2");
-    MCHK(m, dg::cnn::dw_reduce(2, m->dw_part, kDwGroups, m->grads + kW2, m->stream), "dw2 reduce");
-    MCHK(m, dg::cnn::db(dZ2, (long long)c2, 32, 32, m->db_part, kDbBlocks, m->grads + kB2, m->stream), "db2");
+    MCHK(m, dg::cnn::dw(2, B, d1, m->ws[WS_X1].p, dZ2, m->dw_part, kDwGroups, m->grads + kW2, m->stream), "dw2");
     MCHK(m, dg::cnn::conv(2, dg::cnn::CONV_BWD, B, d2, dZ2, m->Wt[1], nullptr, nullptr, dZ1, nullptr,
                           (const float *)m->ws[WS_Z1].p, m->stream), "conv2 bwd");
     // layer 1
-    MCHK(m, dg::cnn::dw(1, B, in, m->ws[WS_X0].p, dZ1, m->dw_part, kDwGroups, m->stream), "dw1");
-    MCHK(m, dg::cnn::dw_reduce(1, m->dw_part, kDwGroups, m->grads + kW1, m->stream), "dw1 reduce");
-    MCHK(m, dg::cnn::db(dZ1, (long long)c1, 32, 32, m->db_part, kDbBlocks, m->grads + kB1, m->stream), "db1");
+    MCHK(m, dg::cnn::dw(1, B, in, m->ws[WS_X0].p, dZ1, m->dw_part, kDwGroups, m->grads + kW1, m->stream), "dw1");
     return DG_OK;
 }
 
@@ -446,8 +439,7 @@ int dg_cnn_create(int device, uint64_t seed, dg_cnn **out)
               hipMalloc((void **)&m->grads, kNParams * 4) == hipSuccess &&
               hipMalloc((void **)&m->adam_m, kNParams * 4) == hipSuccess &&
               hipMalloc((void **)&m->adam_v, kNParams * 4) == hipSuccess &&
-              hipMalloc((void **)&m->dw_part, (size_t)kDwGroups * 27 * 32 * 32 * 4) == hipSuccess &&
-              hipMalloc((void **)&m->db_part, (size_t)kDbBlocks * 32 * 4) == hipSuccess;
+              hipMalloc((void **)&m->dw_part, (size_t)kDwGroups * dg::cnn::dw_part_floats * 4) == hipSuccess;
     for (int l = 0; l < 3 && ok; ++l) {
         ok = hipMalloc((void **)&m->bias_pad[l], 32 * 4) == hipSuccess &&
              hipMemset(m->bias_pad[l], 0, 32 * 4) == hipSuccess &&
@@ -489,7 +481,7 @@ void dg_cnn_destroy(dg_cnn *m)
     if (m->stream) (void)hipStreamSynchronize(m->stream);
     for (int b = 0; b < 2; ++b)
         if (m->graph[b]) (void)hipGraphExecDestroy(m->graph[b]);
-    float *fs[] = {m->params, m->grads, m->adam_m, m->adam_v, m->dw_part, m->db_part, m->tmp,
+    float *fs[] = {m->params, m->grads, m->adam_m, m->adam_v, m->dw_part, m->tmp,
                    m->bias_pad[0], m->bias_pad[1], m->bias_pad[2]};
     for (float *f : fs)
         if (f) (void)hipFree(f);

@@ -244,6 +244,25 @@ inline emu_f32x4 __builtin_amdgcn_mfma_f32_16x16x32_bf16(emu_bf16x8 a, emu_bf16x
     emu::sync();
     return d;
 }
+// Transposed LDS read of 16-bit elements: the 16 lanes of a group address 4
+// rows of 16 elements (lanes 4r .. 4r+3 the 4-element chunks of row r); lane i
+// receives element i of the 4 rows.
+typedef __bf16 emu_bf16x4 __attribute__((ext_vector_type(4)));
+inline emu_bf16x4 __builtin_amdgcn_ds_read_tr16_b64_v4bf16(const emu_bf16x4 *p)
+{
+    const int tid = (int)threadIdx.x, grp = tid & ~15, i = tid & 15;
+    emu::sync();
+    std::memcpy(&emu::xbuf[tid], &p, sizeof(p));
+    emu::sync();
+    emu_bf16x4 out;
+    for (int r = 0; r < 4; ++r) {
+        const emu_bf16x4 *q;
+        std::memcpy(&q, &emu::xbuf[grp + 4 * r + i / 4], sizeof(q));
+        out[r] = (*q)[i % 4];
+    }
+    emu::sync();
+    return out;
+}
 // Direct global->LDS load (size bytes per lane): lane l's bytes land at
 // lds + size * l, visible once the issuing wave waits and the block syncs.
 template <typename P> inline void __builtin_amdgcn_global_load_lds(const void *src, P *lds, int size, int, int)
