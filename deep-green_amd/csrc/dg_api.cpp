@@ -219,9 +219,7 @@ namespace dg {
 
 // Workgroup tiling of a grid: tile_y rows (4, 8, 16; FP64 4, 8), chunk_x
 // x-planes per workgroup (0: the longest chunks that still give ~512
-// workgroups -- two resident per CU of a 256-CU device, one wave of
-// workgroups -- and at least 8 planes; long chunks re-read fewer halo
-// planes).
+// workgroups and at least 8 planes; a single grid's default is choose_tiling's).
 int tile_args(StepArgs &a, int prec, int tile_y, int chunk_x, int *chunk_out)
 {
     if (tile_y != 4 && tile_y != 8 && tile_y != 16) return DG_ERR_INVALID;
@@ -244,6 +242,61 @@ int tile_args(StepArgs &a, int prec, int tile_y, int chunk_x, int *chunk_out)
     a.swizzle = (a.nblocks % 8 == 0) ? 1 : 0;
     if (chunk_out) *chunk_out = lx;
     return DG_OK;
+}
+
+// The tiling of a single grid that the step takes least time for.  A
+// workgroup marches lx planes at c us each after A planes' worth of start-up
+// (the first three planes' loads, nothing hidden); c depends on how many
+// workgroups share a CU (up to the residency of the tile), and workgroups past
+// the device's capacity wait for a round of their own.  c and A were measured
+// per kernel on MI355X (30^3 to 512^3, every tile and chunks of 1 to 64
+// planes) and put the best or a tiling within 6 % of it first on every grid
+// tried.  Step kernel, the ~512-workgroup rule (chunks of at least 8 planes)
+// against this one: FP32 exact 30^3 69 -> 17 us, 64^3 71 -> 27, 256 x 2 x 128
+// 62 -> 21, 192^3 309 -> 267; FP32 fast 192^3 170 -> 129; FP64 192^3 627 -> 508.
+// Fixed values (tile_y, chunk_x not 0) are kept.  Grids that the old rule
+// gave more workgroups than dg_step_noalloc holds keep it; others stay within.
+struct TileCost { int ty, resident; double c[3]; };
+static void choose_tiling(const StepArgs &a, int prec, int fast, int *tile_y, int *chunk_x)
+{
+    static const TileCost kF32Exact[] = {{16, 1, {6.9, 0, 0}}, {8, 2, {4.8, 7.4, 0}}, {4, 3, {4.3, 5.3, 6.4}}};
+    static const TileCost kF32Fast[] = {{8, 2, {2.1, 3.3, 0}}, {16, 1, {3.5, 0, 0}}, {4, 3, {2.1, 2.25, 2.8}}};
+    static const TileCost kF64Exact[] = {{8, 1, {7.2, 0, 0}}, {4, 1, {5.9, 0, 0}}};
+    static const TileCost kF64Fast[] = {{8, 1, {3.5, 0, 0}}, {4, 1, {2.95, 0, 0}}};
+    const TileCost *tab = prec == DG_FP64 ? (fast ? kF64Fast : kF64Exact) : (fast ? kF32Fast : kF32Exact);
+    const int ntab = prec == DG_FP64 ? 2 : 3;
+    const double start = fast ? (prec == DG_FP64 ? 4.4 : 5.8) : 3.0;
+    const long long cus = 256;
+
+    const int ty0 = *tile_y ? *tile_y : ((prec == DG_FP32 && !fast) ? 16 : 8);
+    StepArgs old = a;
+    if (tile_args(old, prec, ty0, *chunk_x, nullptr) != DG_OK || old.nblocks > DG_NOALLOC_MAX_SLOTS) {
+        *tile_y = ty0;
+        return;
+    }
+    double best = -1.0;
+    int best_ty = ty0, best_lx = *chunk_x;
+    for (int k = 0; k < ntab; ++k) {
+        const TileCost &t = tab[k];
+        if (*tile_y && t.ty != *tile_y) continue;
+        const long long yz = (long long)((a.n[1] + t.ty - 1) / t.ty) * ((a.n[2] + 63) / 64);
+        const int most = *chunk_x ? 1 : a.n[0];
+        for (int nbx = 1, lx_last = 0; nbx <= most; ++nbx) {
+            int lx = *chunk_x ? *chunk_x : (a.n[0] + nbx - 1) / nbx;
+            if (lx > a.n[0]) lx = a.n[0];
+            if (lx == lx_last) continue;
+            lx_last = lx;
+            const long long nb = yz * ((a.n[0] + lx - 1) / lx), cap = cus * t.resident;
+            if (nb > DG_NOALLOC_MAX_SLOTS) break;
+            const long long rest = nb % cap;
+            double c = (double)(nb / cap) * t.c[t.resident - 1];
+            if (rest) c += t.c[(rest + cus - 1) / cus - 1];
+            const double cost = (lx + start) * c;
+            if (best < 0 || cost < best * 0.999) { best = cost; best_ty = t.ty; best_lx = lx; }
+        }
+    }
+    *tile_y = best_ty;
+    *chunk_x = best_lx;
 }
 
 // Tiling of a context; drops captured graphs (they bake in the grid).
@@ -300,13 +353,6 @@ int make_args(const dg_config *cfg, StepArgs *out, int *tile_y_out, int *heat_ma
     const size_t el_bytes = cfg->precision == DG_FP64 ? sizeof(double) : sizeof(float);
     if (n3 * el_bytes >= ((size_t)1 << 32)) return bad("a field of this grid exceeds 4 GiB");
     const int prec = cfg->precision, fast = cfg->math == DG_MATH_FAST;
-    // default tile height: 8 rows (two workgroups per CU); FP32 exact math, bound
-    // by its VALU work, takes one 16-row workgroup per CU (fewer halo states per
-    // cell): KHI 512^3 38.9 against 36.0 Gcell/s at 8 rows, FP32-bulk minmod
-    // 256^3 34.3 against 32.3
-    int ty = cfg->tile_y ? cfg->tile_y : ((prec != DG_FP64 && !fast) ? 16 : 8);
-    if (prec == DG_FP64 && ty > 8) ty = 8;
-
     StepArgs a{};
     for (int d = 0; d < 3; ++d) a.n[d] = (int)cfg->n[d];
     // a conducting wall is a wall for the flow; a lower one carries the heat source
@@ -335,7 +381,12 @@ int make_args(const dg_config *cfg, StepArgs *out, int *tile_y_out, int *heat_ma
         a.d2ds = div_const(2.0f * ds);
         a.dds = div_const(ds);
     }
-    if (tile_args(a, prec, ty, cfg->chunk_x, nullptr) != DG_OK) return bad("invalid tile_y or chunk_x");
+    int ty = cfg->tile_y, lx = cfg->chunk_x;
+    if (ty != 0 && ty != 4 && ty != 8 && ty != 16) return bad("invalid tile_y or chunk_x");
+    if (lx < 0) return bad("invalid tile_y or chunk_x");
+    if (prec == DG_FP64 && ty > 8) ty = 8;
+    choose_tiling(a, prec, fast, &ty, &lx);
+    if (tile_args(a, prec, ty, lx, nullptr) != DG_OK) return bad("invalid tile_y or chunk_x");
     *out = a;
     if (tile_y_out) *tile_y_out = ty;
     if (heat_mask_out) *heat_mask_out = heat_mask;
@@ -437,7 +488,8 @@ int create_ctx(const dg_config *cfg, hipStream_t shared_stream, dg_ctx **out, st
     c->args = args;
     c->heat_mask = heat_mask;
     c->nparts_reduce = dg::reduce_blocks(args);
-    if (set_tiling(c, ty, cfg->chunk_x) != DG_OK) { delete c; return failed(DG_ERR_INVALID, "invalid tiling"); }
+    // an ensemble tiles its instances together
+    if (set_tiling(c, ty, shared_stream ? cfg->chunk_x : args.lx) != DG_OK) { delete c; return failed(DG_ERR_INVALID, "invalid tiling"); }
     const size_t n3 = c->n3;
 
     hipError_t e = hipSetDevice(cfg->device);
