@@ -10,8 +10,8 @@
 //                             k = tap * CIN + cin, tap = (dx*3 + dy)*3 + dz;
 //                             A = weights (pre-packed in MFMA fragment order,
 //                             held in VGPRs), B = activations (channels-last)
-//                             read from a ring of input planes in LDS, 16 B
-//                             per lane per k-step (conv_ring_kernel);
+//                             read from input planes in LDS, 16 B per lane
+//                             and k-step (conv_ring_kernel);
 //   weight gradient           D[cout][k] = sum_cells dZ[cell][cout] * X[cell + tap][cin],
 //                             both operands channels-last in LDS, transposed
 //                             by the LDS reads (dw_kernel); one partial per
@@ -31,6 +31,8 @@
 // out = in + 2.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <type_traits>
 
 #include "dg_cnn.h"
 
@@ -55,7 +57,7 @@ __device__ __forceinline__ ErfExp erf_as(float x)
 {
     const float ax = fabsf(x);
     const float t = __builtin_amdgcn_rcpf(fmaf(0.3275911f, ax, 1.0f));
-    const float e = exp2f(-1.44269504088896341f * x * x);
+    const float e = __builtin_amdgcn_exp2f(-1.44269504088896341f * x * x);   // (a denormal one is zero)
     float p = fmaf(1.061405429f, t, -1.453152027f);
     p = fmaf(p, t, 1.421413741f);
     p = fmaf(p, t, -0.284496736f);
@@ -94,33 +96,20 @@ __device__ __forceinline__ bf16x8 zero8()
     return v;
 }
 
-template <int COUT> struct Mfma;
-template <> struct Mfma<32> {
-    typedef f32x16 acc_t;
-    static constexpr int KSTEP = 16, TILE = 32, NACC = 16;
-    static __device__ __forceinline__ acc_t op(bf16x8 a, bf16x8 b, acc_t c)
-    {
-        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-    }
-    // output channel of accumulator i on lane l
-    static __device__ __forceinline__ int row(int i, int lane) { return 8 * (i / 4) + 4 * (lane / 32) + (i % 4); }
-};
-template <> struct Mfma<16> {
-    typedef f32x4 acc_t;
-    static constexpr int KSTEP = 32, TILE = 16, NACC = 4;
-    static __device__ __forceinline__ acc_t op(bf16x8 a, bf16x8 b, acc_t c)
-    {
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-    }
-    static __device__ __forceinline__ int row(int i, int lane) { return 4 * (lane / 16) + i; }
-};
-
+// As convolutions the layers use v_mfma_f32_16x16x32_bf16: a k-step is 32
+// consecutive k of one x tap, i.e. TPS (y, z) taps of all CIN channels, and a
+// wave computes 16 of the COUT output channels.
 template <int CIN, int COUT> struct ConvCfg {
-    static constexpr int KSTEP = Mfma<COUT>::KSTEP;
-    static constexpr int KS = (27 * CIN + KSTEP - 1) / KSTEP;   // k-steps
-    static constexpr int TILE = Mfma<COUT>::TILE;               // cells per MFMA
-    static constexpr int NT = 64 / TILE;                        // cell tiles per wave
-    static constexpr int WAVE_CELLS = 64;
+    static constexpr int TPS = 32 / CIN;               // (y, z) taps per k-step
+    static constexpr int KS = (9 + TPS - 1) / TPS;     // k-steps per input plane
+    static constexpr int CG = COUT / 16;               // groups of output channels
+    static constexpr int WAVES = CIN == 8 ? 16 : 8;    // one workgroup per CU
+    static constexpr int EU = WAVES / 4, THREADS = 64 * WAVES;
+    static constexpr int NT = 16 * CG / WAVES;         // 16-cell tiles per wave (256 cells per workgroup)
+    // 32 -> 32 has the registers for 2 activation fragments in flight and for half
+    // of a thread's share of the next plane at a time, 16 -> 32 for half a share;
+    // otherwise they spill (204 us instead of 155)
+    static constexpr int DEPTH = KS * NT == 36 ? 2 : 4, PARTS = CIN == 16 || KS * NT == 36 ? 2 : 1;
 };
 
 // ---------------------------------------------------------- conv (MFMA) --
@@ -129,27 +118,33 @@ template <int CIN, int COUT> struct ConvCfg {
 // EPI_OUT16: X = bf16(acc + b) (the output layer for the learned step's correction).
 enum { EPI_TRAIN = 0, EPI_INFER = 1, EPI_OUT = 2, EPI_BWD = 3, EPI_OUT16 = 4 };
 
-// ------------------------------------------------ conv (MFMA, LDS ring) --
-// The same convolutions with the activations staged in LDS.  A workgroup
-// (4 waves, one per SIMD) owns a rectangle of RY x RZ output (y, z)
-// positions, flattened row-major (at most 256: 64 per wave, NT MFMA tiles of
-// TILE positions), and marches it along x over a chunk of output planes.
-// Output plane x reads the input planes x - PAD + {0, 1, 2}; they sit in a
-// ring of 4 LDS slots, and the plane needed next is copied into the fourth
-// slot while the current plane is computed (one barrier per plane; its loads
-// are issued before the plane's MFMAs and written to LDS after them).  A slot
-// holds (RY + 2) rows of RING_ROWP cells; a cell
-// is CIN bf16 channels in 16-B chunks, padded by one chunk for CIN >= 16 so
-// that the 128-bit reads of consecutive cells hit distinct banks.  Cells
-// outside the input box load zeros (the full convolution's padding).  The
-// weights stay in VGPRs for the whole kernel, so LDS carries only the
-// activations: one 1-KB read per MFMA.
-constexpr int RING_WAVES = 4;
-constexpr int RING_POS = 64 * RING_WAVES;   // output positions per workgroup plane
-constexpr int RING_ROWP = 48;               // cells per LDS row: RZ + 2 <= RING_ROWP
-constexpr int RING_RMAX = 9;                // LDS rows per slot: RY + 2 <= RING_RMAX
-constexpr int RING_SLOTS = 4;
-constexpr int RING_DEPTH = 3;               // k-steps of B operands loaded ahead
+// --------------------------------------------- conv (MFMA, LDS planes) --
+// The same convolutions with the activations staged in LDS.  A workgroup owns
+// a rectangle of ry x rz output (y, z) positions, flattened row-major (at most
+// 256 in tiles of 16, split over the waves; with 32 output channels a wave takes
+// 16 of them), and marches the INPUT planes of a chunk along
+// x.  Input plane j feeds the output planes j, j - 1 and j - 2 (x taps 0, 1,
+// 2), whose accumulators are all in registers: every activation fragment read
+// from LDS is used by three MFMAs, and only two plane slots are needed, one
+// read while the next plane is loaded to registers (before the MFMAs) and
+// stored (after them), one barrier per plane.  A slot holds (ry + 2) rows of
+// RING_ROWP cells; a cell is CIN bf16 channels in 16-B chunks, padded by one
+// chunk for CIN >= 16 so that the 128-bit reads of consecutive cells hit
+// distinct banks.  Cells outside the input box load zeros (the full
+// convolution's padding).  The weights stay in VGPRs.
+// Two waves per SIMD (four with CIN 8) run the matrix cores under each other's
+// epilogues; the epilogue of a finished plane (GELU) is spread one value at a
+// time over the next plane's k-steps.  Bound by instruction issue: an MFMA
+// keeps the SIMD's VALU from issuing for some 10 of its 16 cycles, and with 32
+// outputs the epilogues take as long as the MFMAs.  An activation fragment per
+// MFMA (outputs gathered from four slots, one wave per SIMD), as before, was
+// bound by LDS and overlapped nothing.  Learned step of 128^3, layers 1-3: 124,
+// 204, 126 -> 85, 155, 59 us; training batch of 8 crops of 32^3, layers 1-3
+// forward 39, 47, 30 -> 25, 31, 17, input gradients of layers 2 and 3 80, 39 ->
+// 50, 30.
+constexpr int RING_POS = 256;               // output positions per workgroup plane
+constexpr int RING_ROWP = 48;               // cells per LDS row: rz + 2 <= RING_ROWP
+constexpr int RING_RMAX = 10;               // LDS rows per slot: ry + 2 <= RING_RMAX
 
 struct RingGeom {
     ConvGeom g;
@@ -162,89 +157,58 @@ struct RingGeom {
 template <int CIN> struct RingCell {
     static constexpr int NC = CIN / 8;                   // 16-B chunks of channels per cell
     static constexpr int CS = NC == 1 ? 1 : NC + 1;      // chunk stride of a cell
-    static constexpr int CHUNKS = RING_RMAX * RING_ROWP * CS;
-    static constexpr int BLOCKS = (CHUNKS + 63) / 64;    // 1-KB blocks (one load instruction per wave)
-    static constexpr int SLOT = BLOCKS * 1024;           // bytes per slot
+    static constexpr int SLOT = RING_RMAX * RING_ROWP * CS * 16;   // bytes per slot
 };
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // zeros for the cells outside the input box (never written)
 static __device__ __attribute__((aligned(16))) uint32_t ring_zero[4];
 
-// Filling a slot with input plane xi of batch item b (rows y0 .. y0 + rows - 1,
-// cells z0 .. z0 + cells - 1): each thread loads its share of 16-B chunks into
-// registers (fill_load, at the top of a plane) and writes them to LDS
-// (fill_store, after the plane's MFMAs), so the loads' latency hides under
-// the MFMAs and the LDS reads keep exact wait counts.
-template <int CIN> struct RingFill {
-    static constexpr int NC = CIN / 8;
-    static constexpr int PER = (RING_RMAX * RING_ROWP * NC + 64 * RING_WAVES - 1) / (64 * RING_WAVES);
-};
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
-template <int CIN>
-__device__ __forceinline__ void fill_load(u32x4 (&v)[RingFill<CIN>::PER], const bf16 *__restrict__ X,
-                                          const ConvGeom &g, int b, int xi, int y0, int z0, int rows, int cells,
-                                          int tid)
+// Computed here: an index of which no 64-bit address is kept across the planes,
+// or a value that is not sunk into the branch that stores it.
+template <typename T> __device__ __forceinline__ T opaque(T v)
 {
-    typedef RingFill<CIN> F;
-    const bool xin = xi >= 0 && xi < g.in[0];
-    const long long pbase = ((long long)b * g.in[0] + xi) * g.in[1];
-#pragma unroll
-    for (int k = 0; k < F::PER; ++k) {
-        const int idx = k * 64 * RING_WAVES + tid;
-        const int cell = idx / F::NC, q = idx % F::NC;
-        const int r = cell / RING_ROWP, c = cell % RING_ROWP;
-        const int yi = y0 + r, zi = z0 + c;
-        const bool in = xin && r < rows && c < cells && yi >= 0 && yi < g.in[1] && zi >= 0 && zi < g.in[2];
-        const u32x4 *src = in ? reinterpret_cast<const u32x4 *>(X + ((pbase + yi) * g.in[2] + zi) * CIN + q * 8)
-                              : reinterpret_cast<const u32x4 *>(ring_zero);
-        v[k] = *src;
-    }
-}
-
-template <int CIN>
-__device__ __forceinline__ void fill_store(char *slot, const u32x4 (&v)[RingFill<CIN>::PER], int rows, int cells,
-                                           int tid)
-{
-    typedef RingFill<CIN> F;
-#pragma unroll
-    for (int k = 0; k < F::PER; ++k) {
-        const int idx = k * 64 * RING_WAVES + tid;
-        const int cell = idx / F::NC, q = idx % F::NC;
-        const int r = cell / RING_ROWP, c = cell % RING_ROWP;
-        if (r < rows && c < cells)
-            *reinterpret_cast<u32x4 *>(slot + (cell * RingCell<CIN>::CS + q) * 16) = v[k];
-    }
+#ifdef __AMDGCN__
+    asm volatile("" : "+v"(v));
+#endif
+    return v;
 }
 
 template <int CIN, int COUT, int EPI, int PAD>
-__global__ void __launch_bounds__(64 * RING_WAVES) __attribute__((amdgpu_waves_per_eu(1, 1)))
+__global__ void __launch_bounds__((ConvCfg<CIN, COUT>::THREADS))
+    __attribute__((amdgpu_waves_per_eu((ConvCfg<CIN, COUT>::EU), (ConvCfg<CIN, COUT>::EU))))
 conv_ring_kernel(const RingGeom rg, const bf16 *__restrict__ X, const bf16x8 *__restrict__ Wp,
                  const float *__restrict__ bias, float *__restrict__ Zout, bf16 *__restrict__ Xout,
                  float *__restrict__ Yout, const float *__restrict__ Zprev)
 {
     typedef ConvCfg<CIN, COUT> C;
-    typedef Mfma<COUT> M;
     typedef RingCell<CIN> RC;
-    constexpr int NT = C::NT;
-    // a k-step lies inside one tap unless CIN < KSTEP (then each lane group has its own tap)
-    constexpr bool ALIGNED = CIN % C::KSTEP == 0;
-    static_assert(ALIGNED || (CIN == 8 && C::KSTEP == 16), "k-step layout");
-    __shared__ __attribute__((aligned(1024))) char ring[RING_SLOTS * RC::SLOT];
+    constexpr int NT = C::NT, KS = C::KS;
+    __shared__ __attribute__((aligned(16))) char ring[2 * RC::SLOT];
 
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int col = lane % C::TILE, part = lane / C::TILE;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int cg = wave % C::CG, pg = wave / C::CG;
+    const int col = lane & 15, part = lane >> 4;
     const ConvGeom &g = rg.g;
 
-    bf16x8 wa[C::KS];
+    bf16x8 wa[KS][3];
 #pragma unroll
-    for (int s = 0; s < C::KS; ++s) wa[s] = Wp[s * 64 + lane];
-    // this lane's output channels' biases (no memory wait in the epilogue)
-    float bv[M::NACC];
+    for (int s = 0; s < KS; ++s)
 #pragma unroll
-    for (int gq = 0; gq < M::NACC / 4; ++gq)
+        for (int dx = 0; dx < 3; ++dx) wa[s][dx] = Wp[((cg * KS + s) * 3 + dx) * 64 + lane];
+    const int ch = 16 * cg + 4 * part;   // this lane's four output channels
+    f32x4 bv = {0, 0, 0, 0};             // their biases: the sums start there
+    if (EPI != EPI_BWD) bv = *reinterpret_cast<const f32x4 *>(bias + ch);
+    // byte offset of this lane's 8 channels of k-step s from its cell: with CIN 32
+    // a constant, with less the lane groups read different taps (past the last:
+    // that one again, with zero weights)
+    int po[KS];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) bv[4 * gq + q] = EPI == EPI_BWD ? 0.0f : bias[M::row(4 * gq, lane) + q];
+    for (int s = 0; s < KS; ++s) {
+        const int tap = C::TPS == 1 ? s : min(s * C::TPS + part / RC::NC, 8);
+        po[s] = (tap / 3 * RING_ROWP + tap % 3) * RC::CS * 16;
+    }
 
     const int RY = rg.ry, RZ = rg.rz, npos = RY * RZ;
     const int o0 = g.out[0], o1 = g.out[1], o2 = g.out[2];
@@ -255,139 +219,160 @@ conv_ring_kernel(const RingGeom rg, const bf16 *__restrict__ X, const bf16x8 *__
         const int xc = (int)(r % rg.nxc);
         const int b = (int)(r / rg.nxc);
         const int y0 = iy * RY, z0 = iz * RZ;
-        const int xs = xc * rg.cx, xe = min(xs + rg.cx, o0);
+        const int xs = xc * rg.cx, n = min(rg.cx, o0 - xs);   // output planes of the item
 
-        // this lane's positions: LDS byte offset within a slot, output (y, z) index
+        // this lane's positions: LDS byte offset (of the plane's slot), output (y, z) index
         int lb[NT], oyz[NT];
         bool ok[NT];
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-            const int p = (wave * NT + t) * C::TILE + col;
+            const int p = (pg * NT + t) * 16 + col;
             const int pp = p < npos ? p : 0;
             const int py = pp / RZ, pz = pp - py * RZ;
             ok[t] = p < npos && y0 + py < o1 && z0 + pz < o2;
-            lb[t] = (py * RING_ROWP + pz) * RC::CS * 16 + (ALIGNED ? part * 16 : 0);
-            oyz[t] = (y0 + py) * o2 + z0 + pz;
+            lb[t] = ((py * RING_ROWP + pz) * RC::CS + part % RC::NC) * 16;
+            oyz[t] = ok[t] ? (y0 + py) * o2 + z0 + pz : 0;
         }
 
-        // prologue: the first three input planes
-        u32x4 fv[RingFill<CIN>::PER];
+        // Staging of an input plane: each thread loads its 16-B chunks to registers
+        // and stores them after the plane's MFMAs (PARTS 2: in halves, each after
+        // half of them).  off: chunk in the plane, -1 for zeros (outside the box, or
+        // cells that no output needs).
+        constexpr int CHUNKS = RING_RMAX * RING_ROWP * RC::NC, PER = (CHUNKS + C::THREADS - 1) / C::THREADS;
+        static_assert(C::THREADS % RC::NC == 0, "a thread's chunks are one channel group");
+        constexpr int PARTS = C::PARTS, PART = (PER + PARTS - 1) / PARTS;
+        u32x4 fv[PART];
+        int off[PER];
 #pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            fill_load<CIN>(fv, X, g, b, xs + j - PAD, y0 - PAD, z0 - PAD, RY + 2, RZ + 2, threadIdx.x);
-            fill_store<CIN>(ring + ((xs + j) & 3) * RC::SLOT, fv, RY + 2, RZ + 2, threadIdx.x);
+        for (int k = 0; k < PER; ++k) {
+            const int cell = (k * C::THREADS + (int)threadIdx.x) / RC::NC, fy = cell / RING_ROWP, fz = cell % RING_ROWP;
+            const int yi = y0 - PAD + fy, zi = z0 - PAD + fz;
+            const bool in = fy < RY + 2 && fz < RZ + 2 && yi >= 0 && yi < g.in[1] && zi >= 0 && zi < g.in[2];
+            off[k] = in ? (yi * g.in[2] + zi) * RC::NC + (int)threadIdx.x % RC::NC : -1;
+        }
+        auto load_part = [&](int j, int h) {
+            const int xi = xs + j - PAD;
+            const bool xin = xi >= 0 && xi < g.in[0];
+            const u32x4 *src = reinterpret_cast<const u32x4 *>(X) +
+                               ((long long)b * g.in[0] + (xin ? xi : 0)) * g.in[1] * g.in[2] * RC::NC;
+#pragma unroll
+            for (int k = h * PART; k < PER && k < (h + 1) * PART; ++k) {
+                const int o = opaque(off[k]);
+                fv[k - h * PART] = *(xin && o >= 0 ? src + o : reinterpret_cast<const u32x4 *>(ring_zero));
+            }
+        };
+        const int dst = ((int)threadIdx.x / RC::NC * RC::CS + (int)threadIdx.x % RC::NC) * 16;
+        auto store_part = [&](int j, int h) {
+            char *slot = ring + (j & 1) * RC::SLOT + dst;
+#pragma unroll
+            for (int k = h * PART; k < PER && k < (h + 1) * PART; ++k)
+                if ((k + 1) * C::THREADS <= CHUNKS || k * C::THREADS + (int)threadIdx.x < CHUNKS)
+                    *reinterpret_cast<u32x4 *>(slot + k * (C::THREADS / RC::NC * RC::CS * 16)) = fv[k - h * PART];
+        };
+#pragma unroll
+        for (int h = 0; h < PARTS; ++h) {
+            load_part(0, h);
+            store_part(0, h);
         }
         __syncthreads();
 
-        // The epilogue of plane x runs in slices between the k-steps of plane
-        // x + 1 (no store waits at the plane's end); the last plane's runs
-        // after the loop.
-        constexpr int NEPI = NT * (M::NACC / 4);
-        auto epilogue = [&](const typename M::acc_t *A, long long mb, int e) {
-            const int t = e / (M::NACC / 4), gq = e % (M::NACC / 4);
-            if (!ok[t]) return;
-            const long long m = mb + oyz[t];
-            const int ch = M::row(4 * gq, lane);
-            float v[4];
+        // accumulators of the output planes j (0), j - 1 (1) and j - 2 (2); prv:
+        // the plane finished before, its epilogue pending
+        f32x4 acc[3][NT], prv[NT];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) v[q] = A[t][4 * gq + q];
-            if (EPI == EPI_BWD) {
-                const f32x4 zp = *reinterpret_cast<const f32x4 *>(Zprev + m * COUT + ch);
-#pragma unroll
-                for (int q = 0; q < 4; ++q) v[q] *= gelu_grad(zp[q]);
-            } else {
-#pragma unroll
-                for (int q = 0; q < 4; ++q) v[q] += bv[4 * gq + q];
-            }
-            if (EPI == EPI_TRAIN) {
-                f32x4 z;
-#pragma unroll
-                for (int q = 0; q < 4; ++q) z[q] = v[q];
-                *reinterpret_cast<f32x4 *>(Zout + m * COUT + ch) = z;
-            }
+        for (int t = 0; t < NT; ++t) acc[0][t] = acc[1][t] = acc[2][t] = prv[t] = f32x4{0, 0, 0, 0};
+        const long long plane_cells = (long long)o1 * o2;
+        const long long mb0 = ((long long)b * o0 + xs) * plane_cells;
+
+        // value q of tile t of the pending plane (output index mb of y = z = 0); the
+        // last of a tile stores its four
+        float ev[4];
+        f32x4 zp[2];   // EPI_BWD: gelu' arguments of this tile and the next
+        auto load_z = [&](long long mb, int t) {
+            if (EPI == EPI_BWD && t < NT)
+                zp[t & 1] = *reinterpret_cast<const f32x4 *>(Zprev + (mb + opaque(oyz[t])) * COUT + ch);
+        };
+        auto epilogue = [&](long long mb, int t, int q) {
+            if (q == 0) load_z(mb, t + 1);
+            const float v = EPI == EPI_BWD ? prv[t][q] * gelu_grad(zp[t & 1][q]) : prv[t][q] + bv[q];
+            if (EPI == EPI_TRAIN) prv[t][q] = v;
+            ev[q] = opaque(EPI == EPI_TRAIN || EPI == EPI_INFER ? gelu(v) : v);
+            if (q != 3 || !ok[t]) return;
+            const long long m = mb + opaque(oyz[t]);
+            if (EPI == EPI_TRAIN) *reinterpret_cast<f32x4 *>(Zout + m * COUT + ch) = prv[t];
             if (EPI == EPI_OUT) {
-                f32x4 y;
-#pragma unroll
-                for (int q = 0; q < 4; ++q) y[q] = v[q];
-                *reinterpret_cast<f32x4 *>(Yout + m * COUT + ch) = y;
+                *reinterpret_cast<f32x4 *>(Yout + m * COUT + ch) = f32x4{ev[0], ev[1], ev[2], ev[3]};
             } else {
                 bf16x4 xo;
 #pragma unroll
-                for (int q = 0; q < 4; ++q) xo[q] = (bf16)(EPI == EPI_BWD || EPI == EPI_OUT16 ? v[q] : gelu(v[q]));
+                for (int i = 0; i < 4; ++i) xo[i] = (bf16)ev[i];
                 *reinterpret_cast<bf16x4 *>(Xout + m * COUT + ch) = xo;
             }
         };
-        const long long plane_cells = (long long)o1 * o2;
-        typename M::acc_t prv[NT];
-        long long pmb = -1;   // output index of (plane of prv, y = z = 0); -1: none pending
 
-        for (int x = xs; x < xe; ++x) {
-            const bool more = x + 1 < xe;
-            if (more) fill_load<CIN>(fv, X, g, b, x + 3 - PAD, y0 - PAD, z0 - PAD, RY + 2, RZ + 2, threadIdx.x);
-            const char *sb[3];
-#pragma unroll
-            for (int dx = 0; dx < 3; ++dx) sb[dx] = ring + ((x + dx) & 3) * RC::SLOT;
-
-            typename M::acc_t acc[NT];
-#pragma unroll
-            for (int t = 0; t < NT; ++t)
-#pragma unroll
-                for (int i = 0; i < M::NACC; ++i) acc[t][i] = 0.0f;
-
-            // B operand of k-step s for tile t (8 channels of one tap of this lane's position)
-            auto load_b = [&](int s, int t) -> bf16x8 {
-                if (ALIGNED) {
-                    const int k = s * C::KSTEP, tap = k / CIN, q = (k % CIN) / 8;
-                    const int dx = tap / 9, dy = (tap / 3) % 3, dz = tap % 3;
-                    const int off = ((dy * RING_ROWP + dz) * RC::CS + q) * 16;
-                    return *reinterpret_cast<const bf16x8 *>(sb[dx] + lb[t] + off);
-                } else {
-                    // CIN 8, KSTEP 16: lanes of part 0 read tap 2s, part 1 tap 2s + 1 (zero past tap 26)
-                    const int ta = 2 * s, tb = 2 * s + 1;
-                    const int offa = ((ta / 3) % 3 * RING_ROWP + ta % 3) * 16;
-                    const int offb = ((tb / 3) % 3 * RING_ROWP + tb % 3) * 16;
-                    const char *pa = sb[ta / 9] + lb[t] + offa;
-                    if (tb >= 27) return part == 0 ? *reinterpret_cast<const bf16x8 *>(pa) : zero8();
-                    const char *pb = sb[tb / 9] + lb[t] + offb;
-                    return *reinterpret_cast<const bf16x8 *>(part == 0 ? pa : pb);
-                }
+        // Input plane j with the x taps of MASK; PENDING: the epilogue of output
+        // plane j - 3 along with it.
+        auto plane = [&](auto mask, auto pending, int j) {
+            constexpr int MASK = decltype(mask)::value;
+            constexpr bool PENDING = decltype(pending)::value;
+            const bool more = j < n + 1;
+            const long long mb = mb0 + (long long)(j - 3) * plane_cells;
+            if (PENDING) load_z(mb, 0);
+            if (more) load_part(j + 1, 0);
+            constexpr int STEPS = KS * NT;
+            constexpr int VPS = (4 * NT + STEPS - 1) / STEPS;        // epilogue values per step,
+            constexpr int EVERY = VPS > 1 ? 1 : STEPS / (4 * NT);    // or steps per value
+            auto load_b = [&](int f) {
+                return *reinterpret_cast<const bf16x8 *>(ring + lb[f % NT] + po[f / NT]);
             };
-            // B operands of RING_DEPTH k-steps in flight (LDS latency under the MFMAs);
-            // the scheduling barriers keep the issue order as written
-            bf16x8 bq[RING_DEPTH][NT];
+            bf16x8 bq[C::DEPTH];
 #pragma unroll
-            for (int d = 0; d < RING_DEPTH; ++d)
-                if (d < C::KS)
+            for (int f = 0; f < C::DEPTH; ++f) bq[f] = load_b(f);
 #pragma unroll
-                    for (int t = 0; t < NT; ++t) bq[d][t] = load_b(d, t);
-            // NEPI segments of SEG k-steps, each followed by one epilogue slice
-            constexpr int SEG = (C::KS + NEPI - 1) / NEPI;
+            for (int f = 0; f < STEPS; ++f) {
+                const int s = f / NT, t = f % NT;
+                const bf16x8 bf = bq[f % C::DEPTH];
 #pragma unroll
-            for (int e = 0; e < NEPI; ++e) {
-#pragma unroll
-                for (int j = 0; j < SEG; ++j) {
-                    const int s = e * SEG + j;
-                    if (s < C::KS) {
-#pragma unroll
-                        for (int t = 0; t < NT; ++t) acc[t] = M::op(wa[s], bq[s % RING_DEPTH][t], acc[t]);
-                        if (s + RING_DEPTH < C::KS)
-#pragma unroll
-                            for (int t = 0; t < NT; ++t) bq[s % RING_DEPTH][t] = load_b(s + RING_DEPTH, t);
-                        __builtin_amdgcn_sched_barrier(0);
+                for (int dx = 2; dx >= 0; --dx)
+                    if (MASK >> dx & 1) {
+                        const f32x4 c = s ? acc[dx][t] : dx ? acc[dx - 1][t] : f32x4{0, 0, 0, 0};
+                        acc[dx][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[s][dx], bf, c, 0, 0, 0);
                     }
+                if (f + C::DEPTH < STEPS) bq[f % C::DEPTH] = load_b(f + C::DEPTH);
+                if (PENDING && f % EVERY == 0)
+#pragma unroll
+                    for (int v = f / EVERY * VPS; v < (f / EVERY + 1) * VPS; ++v)
+                        if (v < 4 * NT) epilogue(mb, v / 4, v % 4);
+                __builtin_amdgcn_sched_barrier(0);
+                if (PARTS == 2 && f == STEPS / 2 && more) {   // the other slot is free since the last barrier
+                    store_part(j + 1, 0);
+                    load_part(j + 1, 1);
                 }
-                if (pmb >= 0) epilogue(prv, pmb, e);
             }
 #pragma unroll
-            for (int t = 0; t < NT; ++t) prv[t] = acc[t];
-            pmb = ((long long)b * o0 + x) * plane_cells;
-            // the slot of plane x - 1 is free since the last barrier
-            if (more) fill_store<CIN>(ring + ((x + 3) & 3) * RC::SLOT, fv, RY + 2, RZ + 2, threadIdx.x);
+            for (int t = 0; t < NT; ++t) {
+                prv[t] = acc[2][t];
+                lb[t] += j & 1 ? -RC::SLOT : RC::SLOT;
+            }
+            if (more) store_part(j + 1, PARTS - 1);
             __syncthreads();
+        };
+        typedef std::integral_constant<bool, true> yes;
+        typedef std::integral_constant<bool, false> no;
+        if (n > 2) {
+            plane(std::integral_constant<int, 1>{}, no{}, 0);
+            plane(std::integral_constant<int, 3>{}, no{}, 1);
+            plane(std::integral_constant<int, 7>{}, no{}, 2);
+            for (int j = 3; j < n; ++j) plane(std::integral_constant<int, 7>{}, yes{}, j);
+            plane(std::integral_constant<int, 6>{}, yes{}, n);
+            plane(std::integral_constant<int, 4>{}, yes{}, n + 1);
+        } else {   // x taps without an output plane accumulate in registers that nothing reads
+            for (int j = 0; j < 3; ++j) plane(std::integral_constant<int, 7>{}, no{}, j);
+            if (n == 2) plane(std::integral_constant<int, 4>{}, yes{}, 3);
         }
-        if (pmb >= 0)
+        load_z(mb0 + (n - 1) * plane_cells, 0);
 #pragma unroll
-            for (int e = 0; e < NEPI; ++e) epilogue(prv, pmb, e);
+        for (int v = 0; v < 4 * NT; ++v) epilogue(mb0 + (n - 1) * plane_cells, v / 4, v % 4);
     }
 }
 
@@ -564,7 +549,7 @@ dw_kernel(const DwGeom dg, const bf16 *__restrict__ X, const bf16 *__restrict__ 
 #pragma unroll
                         for (int i = 0; i < 8; ++i) bv[i] = one ? (bf16)1.0f : bv[i];
                     }
-                    acc[t] = Mfma<32>::op(a, bv, acc[t]);
+                    acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, bv, acc[t], 0, 0, 0);
                 }
             }
             if (more) { store_x(x + 3); store_z(x + 1); }
@@ -606,7 +591,7 @@ dw_kernel(const DwGeom dg, const bf16 *__restrict__ X, const bf16 *__restrict__ 
         for (int t = 0; t < TPW; ++t)
 #pragma unroll
             for (int q = 0; q < 4; ++q)
-                *reinterpret_cast<f32x4 *>(P + ((tg * TPW + t) * 32 + lane % 32) * 32 + Mfma<32>::row(4 * q, lane)) =
+                *reinterpret_cast<f32x4 *>(P + ((tg * TPW + t) * 32 + lane % 32) * 32 + 8 * q + 4 * (lane / 32)) =
                     f32x4{acc[t][4 * q], acc[t][4 * q + 1], acc[t][4 * q + 2], acc[t][4 * q + 3]};
     }
 }
@@ -643,15 +628,15 @@ __global__ void pack_kernel(const float *__restrict__ W, int cin_real, int cout_
 {
     // as a convolution: CI input channels (padded CIP), CO output channels (padded COP)
     const int CIP = transpose ? cout_pad : cin_pad, COP = transpose ? cin_pad : cout_pad;
-    const int kstep = COP == 32 ? 16 : 32, tile = COP == 32 ? 32 : 16;
-    const int ks = (27 * CIP + kstep - 1) / kstep;
+    const int tps = 32 / CIP, ks = (9 + tps - 1) / tps;
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= ks * 64 * 8) return;
-    const int i = e % 8, lane = (e / 8) % 64, s = e / 512;
-    const int k = s * kstep + (lane / tile) * 8 + i, n = lane % tile;
-    const int tap = k / CIP, c = k % CIP;
+    if (e >= COP / 16 * ks * 3 * 64 * 8) return;
+    const int i = e % 8, lane = (e / 8) % 64, f = e / 512;
+    const int dx = f % 3, s = f / 3 % ks, cg = f / (3 * ks);
+    const int k = (lane / 16) * 8 + i, n = 16 * cg + lane % 16;
+    const int yz = s * tps + k / CIP, tap = 9 * dx + yz, c = k % CIP;
     float v = 0.0f;
-    if (tap < 27) {
+    if (yz < 9) {
         if (!transpose) {
             if (c < cin_real && n < cout_real) v = W[((size_t)tap * cin_real + c) * cout_real + n];
         } else {
@@ -851,27 +836,38 @@ static int cu_count()
     return n;
 }
 
-// Rectangles of at most RING_POS positions with RZ + 2 <= RING_ROWP and
-// RY + 2 <= RING_RMAX, balanced over the output extents; x chunks so that
-// there are about four work items per CU.
+// Rectangles of at most RING_POS positions with rz + 2 <= RING_ROWP and
+// ry + 2 <= RING_RMAX: those with the least work per plane (a workgroup computes
+// RING_POS positions whatever it owns, and stages the halo); x chunks: the
+// shortest schedule on the CUs, an item costing its planes plus 3.
 static RingGeom ring_geom(const ConvGeom &g)
 {
     RingGeom r;
     r.g = g;
     const int o0 = g.out[0], o1 = g.out[1], o2 = g.out[2];
-    r.nz = (o2 + RING_ROWP - 3) / (RING_ROWP - 2);
-    r.rz = (o2 + r.nz - 1) / r.nz;
-    int ry = RING_POS / r.rz;
-    if (ry > RING_RMAX - 2) ry = RING_RMAX - 2;
-    if (ry > o1) ry = o1;
-    if (ry < 1) ry = 1;
-    r.ny = (o1 + ry - 1) / ry;
-    r.ry = (o1 + r.ny - 1) / r.ny;
-    const long long cols = (long long)g.B * r.ny * r.nz;
-    long long nxc = (4LL * cu_count() + cols - 1) / cols;
-    if (nxc > o0) nxc = o0;
-    if (nxc < 1) nxc = 1;
-    r.cx = (int)((o0 + nxc - 1) / nxc);
+    long long best = -1;
+    const int nz0 = (o2 + RING_ROWP - 3) / (RING_ROWP - 2);
+    for (int nz = nz0; nz <= nz0 + 4 && nz <= o2; ++nz) {
+        const int rz = (o2 + nz - 1) / nz;
+        int ry = RING_POS / rz;
+        if (ry > RING_RMAX - 2) ry = RING_RMAX - 2;
+        if (ry > o1) ry = o1;
+        const int ny = (o1 + ry - 1) / ry;
+        ry = (o1 + ny - 1) / ny;
+        const long long cost = (long long)ny * nz * (4 * RING_POS + (ry + 2) * (rz + 2));
+        if (best < 0 || cost < best) {
+            best = cost;
+            r.ry = ry; r.rz = rz;
+            r.ny = ny; r.nz = (o2 + rz - 1) / rz;
+        }
+    }
+    const long long cols = (long long)g.B * r.ny * r.nz, cus = cu_count();
+    best = -1;
+    r.cx = o0;
+    for (int cx = o0; cx >= 1; --cx) {
+        const long long rounds = (cols * ((o0 + cx - 1) / cx) + cus - 1) / cus, cost = rounds * (cx + 3);
+        if (best < 0 || cost < best) { best = cost; r.cx = cx; }
+    }
     r.nxc = (o0 + r.cx - 1) / r.cx;
     r.items = cols * r.nxc;
     return r;
@@ -885,13 +881,15 @@ int conv(int layer, int mode, int B, const int in[3], const void *X, const void 
     for (int d = 0; d < 3; ++d)
         if (g.out[d] < 1) return -1;
     const RingGeom rg = ring_geom(g);
-    const int blocks = (int)(rg.items < cu_count() ? rg.items : cu_count());
     const bf16 *x = static_cast<const bf16 *>(X);
     const bf16x8 *w = static_cast<const bf16x8 *>(Wp);
     bf16 *xo = static_cast<bf16 *>(Xout);
-#define DG_CONV(CI, CO, E, P)                                                                                 \
-    hipLaunchKernelGGL((conv_ring_kernel<CI, CO, E, P>), dim3(blocks), dim3(64 * RING_WAVES), 0, s, rg, x, w, bias, Z, \
-                       xo, Y, Zprev)
+#define DG_CONV(CI, CO, E, P)                                                                                    \
+    do {                                                                                                         \
+        const long long fit = (long long)cu_count() * (4 * ConvCfg<CI, CO>::EU / ConvCfg<CI, CO>::WAVES);         \
+        hipLaunchKernelGGL((conv_ring_kernel<CI, CO, E, P>), dim3((unsigned)(rg.items < fit ? rg.items : fit)),  \
+                           dim3(ConvCfg<CI, CO>::THREADS), 0, s, rg, x, w, bias, Z, xo, Y, Zprev);               \
+    } while (0)
     if (layer == 1) {
         if (mode == CONV_TRAIN) DG_CONV(8, 32, EPI_TRAIN, 0);
         else if (mode == CONV_INFER) DG_CONV(8, 32, EPI_INFER, 0);
@@ -976,8 +974,8 @@ int pack_elems(int layer, int transpose)
 {
     const int cin_pad = layer == 1 ? 8 : 32, cout_pad = layer == 3 ? 16 : 32;
     const int CIP = transpose ? cout_pad : cin_pad, COP = transpose ? cin_pad : cout_pad;
-    const int kstep = COP == 32 ? 16 : 32;
-    return ((27 * CIP + kstep - 1) / kstep) * 64 * 8;
+    const int tps = 32 / CIP, ks = (9 + tps - 1) / tps;
+    return COP / 16 * ks * 3 * 64 * 8;
 }
 
 int adam(float *w, const float *g, float *m, float *v, int n, float lr, float b1, float b2, float eps, long long t,

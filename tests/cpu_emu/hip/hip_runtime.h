@@ -88,6 +88,7 @@ template <typename T> inline T __shfl_down(T v, unsigned d) { return emu::exch<T
 template <typename T> inline T __shfl_up(T v, unsigned d) { return emu::exch<T>(v, (int)d, 1); }
 template <typename T> inline T __shfl_xor(T v, int m) { return emu::exch<T>(v, m, 2); }
 inline float __builtin_amdgcn_rcpf(float x) { return 1.0f / x; }
+inline float __builtin_amdgcn_exp2f(float x) { return exp2f(x); }
 inline float __builtin_amdgcn_sqrtf(float x) { return std::sqrt(x); }
 inline float __builtin_amdgcn_rsqf(float x) { return 1.0f / std::sqrt(x); }
 inline double __builtin_amdgcn_rcp(double x) { return 1.0 / x; }

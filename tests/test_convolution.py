@@ -1,0 +1,69 @@
+"""The convolutions (conv_ring_kernel) at the edges of their tiling: chunks of
+one, two and three output planes, rows and rectangles that end inside a
+16-cell tile, several rectangles and batch items, against torch (the kernels'
+bfloat16 rounding points; tolerances of the other network tests).  An input
+that is not finite reaches exactly the outputs whose windows hold it: neither
+padded k-steps nor the accumulators of planes that do not exist leak."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+import cnn_reference as ref  # noqa: E402
+from test_cnn_emulation import check_grads, emu_lib, rel  # noqa: E402, F401
+
+
+def network(lib, seed):
+    from deepgreen.learned import FluxCNN
+    m = FluxCNN(seed=seed, lib=lib)
+    p = ref.split(m.get_params())
+    p["b1"] = np.linspace(-0.2, 0.2, 32, dtype=np.float32)
+    p["b3"] = np.linspace(-0.1, 0.1, 15, dtype=np.float32)
+    m.set_params(np.concatenate([np.asarray(p[k], np.float32).reshape(-1) for k, _ in ref.LAYOUT]))
+    return m
+
+
+def run(lib, batch, dims, seed):
+    m = network(lib, seed)
+    rng = np.random.default_rng(seed)
+    x = rng.normal(size=(batch,) + dims + (5,)).astype(np.float32)
+    dy = rng.normal(size=(batch,) + tuple(d - 6 for d in dims) + (15,)).astype(np.float32)
+    y, g = m.forward(x), m.backward(x, dy)
+    net = ref.Net(m.get_params())
+    yr = net.forward(x)
+    (yr * torch.as_tensor(dy)).sum().backward()
+    assert rel(y, yr.detach().numpy()) < 1e-2
+    check_grads(g, net.grads_flat())
+
+
+def run_nonfinite(lib, dims, at):
+    m = network(lib, 4)
+    x = np.random.default_rng(4).normal(size=(1,) + dims + (5,)).astype(np.float32)
+    x[(0,) + at + (2,)] = np.nan
+    bad = ~np.isfinite(m.forward(x)[0]).all(axis=-1)
+    want = np.zeros_like(bad)
+    want[tuple(slice(max(a - 6, 0), a + 1) for a in at)] = True
+    np.testing.assert_array_equal(bad, want)
+
+
+@pytest.mark.parametrize("batch,dims", [(2, (8, 7, 54)), (1, (9, 15, 9))])
+def test_emulated_convolution_tiles(emu_lib, batch, dims):  # noqa: F811
+    run(emu_lib, batch, dims, 5)
+
+
+def test_emulated_nonfinite_input_stays_local(emu_lib):  # noqa: F811
+    run_nonfinite(emu_lib, (9, 10, 9), (8, 0, 8))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,dims", [(1, (7, 7, 7)), (2, (8, 7, 52)), (1, (9, 8, 53)), (1, (10, 16, 22)),
+                                        (3, (11, 15, 54)), (2, (21, 60, 38)), (1, (30, 33, 130)), (40, (7, 9, 8))])
+def test_convolution_tiles(batch, dims):
+    print(f"  convolution {batch} x {dims}", flush=True)
+    run(None, batch, dims, 6)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dims,at", [((9, 10, 9), (8, 0, 8)), ((20, 30, 60), (10, 14, 46)), ((16, 16, 16), (0, 15, 7))])
+def test_nonfinite_input_stays_local(dims, at):
+    print(f"  non-finite input {dims} {at}", flush=True)
+    run_nonfinite(None, dims, at)
