@@ -45,10 +45,18 @@ int conv(int layer, int mode, int B, const int in[3], const void *X, const void 
 constexpr int dw_part_floats = 28 * 32 * 32;
 int dw(int layer, int B, const int in[3], const void *X, const void *dZ, float *partials, int nwg, float *grad,
        hipStream_t s);
-int pack(int layer, int transpose, const float *W, void *Wp, hipStream_t s);
+// The bf16 weights in the convolutions' fragment order (pack_elems elements of
+// a layer; transpose: its input gradient's, layers 2 and 3) and the biases
+// padded to 32.  pack and adam write what the n parameters determine; the
+// padding has to be zero.
+struct Packed {
+    void *w[3], *wt[3];
+    float *bias[3];
+};
+int pack(const float *w, int n, const Packed &P, hipStream_t s);
 int pack_elems(int layer, int transpose);
 int adam(float *w, const float *g, float *m, float *v, int n, float lr, float b1, float b2, float eps, long long t,
-         hipStream_t s);
+         const Packed &P, hipStream_t s);
 // zero (optional): a counter the kernel also sets to 0 (the learned step's
 // fallback count, which saves that step a launch).
 int prep_input(const PrepArgs &a, const float *const *samples, const int *boxes, void *X, hipStream_t s,

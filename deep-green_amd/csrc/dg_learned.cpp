@@ -38,7 +38,7 @@ namespace {
 const int kCin[3] = {5, 32, 32}, kCout[3] = {32, 32, 15};
 const int64_t kW1 = 0, kB1 = kW1 + 27 * 5 * 32, kW2 = kB1 + 32, kB2 = kW2 + 27 * 32 * 32, kW3 = kB2 + 32,
               kB3 = kW3 + 27 * 32 * 15, kNParams = kB3 + 15;
-const int64_t kWoff[3] = {kW1, kW2, kW3}, kBoff[3] = {kB1, kB2, kB3};
+const int64_t kWoff[3] = {kW1, kW2, kW3};
 const int kDwGroups = 256;     // workgroups of the weight-gradient kernels
 const int kLossBlocks = 256;
 const int kGraphSteps = 16;
@@ -125,14 +125,20 @@ void *ws(dg_cnn *m, int k, size_t n)
 
 enum { WS_X0, WS_Z1, WS_X1, WS_Z2, WS_X2, WS_G, WS_T, WS_DG, WS_DZ2, WS_DZ1, WS_Y, WS_BOX, WS_IX1, WS_IX2, WS_IG };
 
+dg::cnn::Packed packed(const dg_cnn *m)
+{
+    dg::cnn::Packed P;
+    for (int l = 0; l < 3; ++l) {
+        P.w[l] = m->Wp[l];
+        P.wt[l] = m->Wt[l];
+        P.bias[l] = m->bias_pad[l];
+    }
+    return P;
+}
+
 int sync_weights(dg_cnn *m)
 {
-    for (int l = 0; l < 3; ++l) {
-        MCHK(m, dg::cnn::pack(l + 1, 0, m->params + kWoff[l], m->Wp[l], m->stream), "pack");
-        if (l > 0) MCHK(m, dg::cnn::pack(l + 1, 1, m->params + kWoff[l], m->Wt[l], m->stream), "pack");
-        MHIP(m, hipMemcpyAsync(m->bias_pad[l], m->params + kBoff[l], kCout[l] * sizeof(float),
-                               hipMemcpyDeviceToDevice, m->stream));
-    }
+    MCHK(m, dg::cnn::pack(m->params, (int)kNParams, packed(m), m->stream), "pack");
     return DG_OK;
 }
 
@@ -165,8 +171,7 @@ int backward(dg_cnn *m, int B, const int in[3])
 {
     const int d1[3] = {in[0] - 2, in[1] - 2, in[2] - 2}, d2[3] = {in[0] - 4, in[1] - 4, in[2] - 4},
               d3[3] = {in[0] - 6, in[1] - 6, in[2] - 6};
-    const size_t c1 = (size_t)B * d1[0] * d1[1] * d1[2], c2 = (size_t)B * d2[0] * d2[1] * d2[2],
-                 c3 = (size_t)B * d3[0] * d3[1] * d3[2];
+    const size_t c1 = (size_t)B * d1[0] * d1[1] * d1[2], c2 = (size_t)B * d2[0] * d2[1] * d2[2];
     void *dZ2 = ws(m, WS_DZ2, c2 * 32 * 2);
     void *dZ1 = ws(m, WS_DZ1, c1 * 32 * 2);
     if (!dZ2 || !dZ1) return mfail(m, DG_ERR_ALLOC, "workspace");
@@ -188,8 +193,8 @@ int adam_update(dg_cnn *m, float lr, float b1, float b2, float eps)
 {
     m->adam_t += 1;
     MCHK(m, dg::cnn::adam(m->params, m->grads, m->adam_m, m->adam_v, (int)kNParams, lr, b1, b2, eps, m->adam_t,
-                          m->stream), "adam");
-    return sync_weights(m);
+                          packed(m), m->stream), "adam");
+    return DG_OK;
 }
 
 // losses: per-block partials of one batch, summed on the host later
@@ -443,8 +448,11 @@ int dg_cnn_create(int device, uint64_t seed, dg_cnn **out)
     for (int l = 0; l < 3 && ok; ++l) {
         ok = hipMalloc((void **)&m->bias_pad[l], 32 * 4) == hipSuccess &&
              hipMemset(m->bias_pad[l], 0, 32 * 4) == hipSuccess &&
-             hipMalloc(&m->Wp[l], dg::cnn::pack_elems(l + 1, 0) * 2) == hipSuccess;
-        if (ok && l > 0) ok = hipMalloc(&m->Wt[l], dg::cnn::pack_elems(l + 1, 1) * 2) == hipSuccess;
+             hipMalloc(&m->Wp[l], dg::cnn::pack_elems(l + 1, 0) * 2) == hipSuccess &&
+             hipMemset(m->Wp[l], 0, dg::cnn::pack_elems(l + 1, 0) * 2) == hipSuccess;
+        if (ok && l > 0)
+            ok = hipMalloc(&m->Wt[l], dg::cnn::pack_elems(l + 1, 1) * 2) == hipSuccess &&
+                 hipMemset(m->Wt[l], 0, dg::cnn::pack_elems(l + 1, 1) * 2) == hipSuccess;
     }
     if (!ok) {
         dg_cnn_destroy(m);

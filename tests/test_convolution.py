@@ -67,3 +67,28 @@ def test_convolution_tiles(batch, dims):
 def test_nonfinite_input_stays_local(dims, at):
     print(f"  non-finite input {dims} {at}", flush=True)
     run_nonfinite(None, dims, at)
+
+
+def run_packed(lib):
+    """The weights that Adam packs as it updates them act as those set anew."""
+    from deepgreen.learned import FluxCNN
+    a, b = network(lib, 7), FluxCNN(seed=8, lib=lib)
+    rng = np.random.default_rng(7)
+    for _ in range(2):
+        a.adam_step(rng.normal(size=a.get_params().size).astype(np.float32), lr=1e-2)
+    b.set_params(a.get_params())
+    x = rng.normal(size=(1, 8, 7, 9, 5)).astype(np.float32)
+    dy = rng.normal(size=(1, 2, 1, 3, 15)).astype(np.float32)
+    np.testing.assert_array_equal(a.forward(x), b.forward(x))
+    np.testing.assert_array_equal(a.backward(x, dy), b.backward(x, dy))
+    net = ref.Net(a.get_params())
+    assert rel(a.forward(x), net.forward(x).detach().numpy()) < 1e-2
+
+
+def test_emulated_adam_packs_the_weights(emu_lib):  # noqa: F811
+    run_packed(emu_lib)
+
+
+@pytest.mark.gpu
+def test_adam_packs_the_weights():
+    run_packed(None)
