@@ -744,49 +744,66 @@ prep_target_kernel(const PrepArgs a, const float *const *__restrict__ samples, c
 // Divergence loss over the L^3 box: P[c][q] = -sum_d (G[c+1][5d+q] - G[c+1-e_d][5d+q])
 // (G on (L+1)^3, index c+1 = face c + e_d/2), loss = mean (P - T)^2 over cells and
 // the 5 components; dG = dloss/dG (bf16, 16 channels, channel 15 zero); per-block
-// partial loss sums.
-__global__ void __launch_bounds__(256)
+// partial loss sums.  A thread needs the errors of its cell and of three
+// neighbours, 40 16-byte loads (L1 and L2) and nothing to hide them but other
+// waves: 1024 threads per block.  8 crops of 32^3: 72 -> 36 us (scalar
+// loads, four errors per component, 256 threads).
+constexpr int LOSS_THREADS = 1024;
+__global__ void __launch_bounds__(LOSS_THREADS)
 loss_kernel(int B, int L, const float *__restrict__ G, const float *__restrict__ T, bf16 *__restrict__ dG,
             double *__restrict__ loss_part)
 {
-    __shared__ double red[256];
+    __shared__ double red[LOSS_THREADS];
     const int Lg = L + 1;
-    const long long perg = (long long)Lg * Lg * Lg, total = perg * B;
+    const uint32_t perg = (uint32_t)Lg * Lg * Lg;
+    const long long total = (long long)perg * B;
     const double N = (double)B * L * L * L * 5;
     const float scale = (float)(2.0 / N);
     double lsum = 0.0;
     for (long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < total;
          e += (long long)gridDim.x * blockDim.x) {
         const int b = (int)(e / perg);
-        long long r = e % perg;
+        uint32_t r = (uint32_t)(e % perg);
         const int gz = (int)(r % Lg); r /= Lg;
         const int gy = (int)(r % Lg);
         const int gx = (int)(r / Lg);
-        // error of cell c = g - 1 (as the +G[c+1] term) and residual helpers
-        auto err = [&](int cx, int cy, int cz, int q) -> float {
-            if (cx < 0 || cy < 0 || cz < 0 || cx >= L || cy >= L || cz >= L) return 0.0f;
-            const long long gb = (long long)b * perg;
-            const long long g0 = gb + (((long long)(cx + 1) * Lg + (cy + 1)) * Lg + (cz + 1));
-            const long long gxm = g0 - (long long)Lg * Lg, gym = g0 - Lg, gzm = g0 - 1;
-            const float P = -((G[g0 * 16 + q] - G[gxm * 16 + q]) + (G[g0 * 16 + 5 + q] - G[gym * 16 + 5 + q]) +
-                              (G[g0 * 16 + 10 + q] - G[gzm * 16 + 10 + q]));
-            const long long t = (((long long)b * L + cx) * L + cy) * L + cz;
-            return P - T[t * 5 + q];
+        // errors of cell c (zero outside the box)
+        auto err = [&](int cx, int cy, int cz, float *out) {
+            if (cx < 0 || cy < 0 || cz < 0 || cx >= L || cy >= L || cz >= L) {
+#pragma unroll
+                for (int q = 0; q < 5; ++q) out[q] = 0.0f;
+                return;
+            }
+            const long long g0 = (long long)b * perg + (((long long)(cx + 1) * Lg + (cy + 1)) * Lg + (cz + 1));
+            const f32x4 *own = reinterpret_cast<const f32x4 *>(G + g0 * 16);
+            const f32x4 *xm = own - (long long)Lg * Lg * 4, *ym = own - (long long)Lg * 4, *zm = own - 4;
+            const f32x4 a0 = own[0], a1 = own[1], a2 = own[2], a3 = own[3];
+            const f32x4 x0 = xm[0], x1 = xm[1], y1 = ym[1], y2 = ym[2], z2 = zm[2], z3 = zm[3];
+            const float gx0[5] = {a0[0], a0[1], a0[2], a0[3], a1[0]}, gx1[5] = {x0[0], x0[1], x0[2], x0[3], x1[0]};
+            const float gy0[5] = {a1[1], a1[2], a1[3], a2[0], a2[1]}, gy1[5] = {y1[1], y1[2], y1[3], y2[0], y2[1]};
+            const float gz0[5] = {a2[2], a2[3], a3[0], a3[1], a3[2]}, gz1[5] = {z2[2], z2[3], z3[0], z3[1], z3[2]};
+            const float *t = T + ((((long long)b * L + cx) * L + cy) * L + cz) * 5;
+#pragma unroll
+            for (int q = 0; q < 5; ++q)
+                out[q] = -((gx0[q] - gx1[q]) + (gy0[q] - gy1[q]) + (gz0[q] - gz1[q])) - t[q];
         };
-        bf16x8 lo = zero8(), hi = zero8();
         const int cx = gx - 1, cy = gy - 1, cz = gz - 1;
+        float e0[5], n[3][5];
+        err(cx, cy, cz, e0);
+        err(cx + 1, cy, cz, n[0]);
+        err(cx, cy + 1, cz, n[1]);
+        err(cx, cy, cz + 1, n[2]);
+        bf16x8 lo = zero8(), hi = zero8();
+#pragma unroll
         for (int q = 0; q < 5; ++q) {
-            const float e0 = err(cx, cy, cz, q);
-            if (cx >= 0 && cy >= 0 && cz >= 0) lsum += (double)e0 * e0;
+            if (cx >= 0 && cy >= 0 && cz >= 0) lsum += (double)e0[q] * e0[q];
             // d/dG[g][5d+q]: -e(c) from cell c = g-1, + e(c + e_d) from cell g-1+e_d
-            const float gx_ = scale * (-e0 + err(cx + 1, cy, cz, q));
-            const float gy_ = scale * (-e0 + err(cx, cy + 1, cz, q));
-            const float gz_ = scale * (-e0 + err(cx, cy, cz + 1, q));
-            const float v[3] = {gx_, gy_, gz_};
+#pragma unroll
             for (int d = 0; d < 3; ++d) {
                 const int ch = 5 * d + q;
-                if (ch < 8) lo[ch] = (bf16)v[d];
-                else hi[ch - 8] = (bf16)v[d];
+                const bf16 v = (bf16)(scale * (-e0[q] + n[d][q]));
+                if (ch < 8) lo[ch] = v;
+                else hi[ch - 8] = v;
             }
         }
         *reinterpret_cast<bf16x8 *>(dG + e * 16) = lo;
@@ -794,7 +811,7 @@ loss_kernel(int B, int L, const float *__restrict__ G, const float *__restrict__
     }
     red[threadIdx.x] = lsum;
     __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
+    for (int s = LOSS_THREADS / 2; s > 0; s >>= 1) {
         if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
         __syncthreads();
     }
@@ -1010,7 +1027,7 @@ int prep_target(const PrepArgs &a, const float *const *samples, const int *boxes
 
 int loss(int B, int L, const float *G, const float *T, void *dG, double *loss_part, int nblk, hipStream_t s)
 {
-    hipLaunchKernelGGL(loss_kernel, dim3(nblk), dim3(256), 0, s, B, L, G, T, static_cast<bf16 *>(dG), loss_part);
+    hipLaunchKernelGGL(loss_kernel, dim3(nblk), dim3(LOSS_THREADS), 0, s, B, L, G, T, static_cast<bf16 *>(dG), loss_part);
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
