@@ -887,6 +887,36 @@ __device__ __forceinline__ void block_partials(double den, int nanf, const doubl
     }
 }
 
+// The same for the max den and NaN flag alone (the five sums are read only
+// after a reduction over a whole state): 8 cross-lane operations with float
+// den, where all seven values in double took 84 at the end of each workgroup.
+template <int NT, typename T>
+__device__ __forceinline__ void block_den(T den, int nanf, double *red, double *P, int tid)
+{
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) {
+        const T other = __shfl_xor(den, off);
+        den = other > den ? other : den;
+        nanf |= __shfl_xor(nanf, off);
+    }
+    constexpr int NW = NT / 64;
+    const int w = tid >> 6, lane = tid & 63;
+    if (lane == 0) {
+        red[w * 8] = (double)den;
+        red[w * 8 + 1] = (double)nanf;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        double d = red[0], n = red[1];
+        for (int ww = 1; ww < NW; ++ww) {
+            d = fmax(d, red[ww * 8]);
+            n = fmax(n, red[ww * 8 + 1]);
+        }
+        P[0] = d;
+        P[1] = n;
+    }
+}
+
 // One tile (TY x 64 columns, planes [bx*lx, min(bx*lx+lx, nx))) of one
 // grid: the whole fused step for those cells; writes the tile's partial
 // (max wave-speed denominator, NaN flag) to partial_out.  Called by the
@@ -1306,9 +1336,8 @@ __device__ __forceinline__ void step_tile(StepLDS<T, TY, FAST> &L, double *red, 
         if (++t > xend) break;
     }
 
-    if constexpr (!BULK) dmaxden = (double)maxden;
-    const double nosums[5] = {0, 0, 0, 0, 0};
-    block_partials<NT>(dmaxden, nanf, nosums, red, partial_out, 0, tid);
+    if constexpr (BULK) block_den<NT>(dmaxden, nanf, red, partial_out, tid);
+    else block_den<NT>(maxden, nanf, red, partial_out, tid);
 }
 
 // Occupancy target: the FP32 kernels fit 128 VGPRs (4 waves per SIMD; exact
@@ -1419,24 +1448,31 @@ reduce_kernel(const StepArgs A, const Fields<const T> U, double *__restrict__ pa
 // cells of ds / den == CFL * ds / max den), conservation sums, and the run
 // clock (main.rs:64-66).  One workgroup of NT threads; fixed reduction
 // order.  mode 0: dt and sums of a fresh state; 1: after a step (advance the
-// clock, new dt); 2: sums only.
+// clock, new dt; the partials hold no sums); 2: sums only.  All latency: the
+// scalars are loaded before the reduction (6.2 -> 3.9 us after a step of 30^3).
 template <typename T, bool BULK, int NT>
 __device__ __forceinline__ void finalize_body(double ds, Scalars *__restrict__ sc, const double *__restrict__ partials,
                                               int np, double cfl, int nan_fallback, int mode, double *red)
 {
     const int tid = threadIdx.x;
-    double den = 0.0, nanf = 0.0, s[5] = {0, 0, 0, 0, 0};
+    double t_now = sc->t;
+    const double dt_now = sc->dt, t_end = sc->t_end;
+    long long steps = sc->steps;
+    const long long max_steps = sc->max_steps;
+    const int active = sc->active;
+    double v[7] = {0, 0, 0, 0, 0, 0, 0};
     for (int i = tid; i < np; i += NT) {
         const double *P = partials + (size_t)i * PARTIAL_STRIDE;
-        den = fmax(den, P[0]);
-        nanf = fmax(nanf, P[1]);
-        for (int q = 0; q < 5; ++q) s[q] += P[2 + q];
+        v[0] = fmax(v[0], P[0]);
+        v[1] = fmax(v[1], P[1]);
+        if (mode != 1)
+            for (int q = 2; q < 7; ++q) v[q] += P[q];
     }
-    double v[7] = {den, nanf, s[0], s[1], s[2], s[3], s[4]};
     for (int off = 32; off >= 1; off >>= 1) {
         v[0] = fmax(v[0], __shfl_xor(v[0], off));
         v[1] = fmax(v[1], __shfl_xor(v[1], off));
-        for (int q = 2; q < 7; ++q) v[q] += __shfl_xor(v[q], off);
+        if (mode != 1)
+            for (int q = 2; q < 7; ++q) v[q] += __shfl_xor(v[q], off);
     }
     if ((tid & 63) == 0)
         for (int q = 0; q < 7; ++q) red[(tid >> 6) * 8 + q] = v[q];
@@ -1447,17 +1483,20 @@ __device__ __forceinline__ void finalize_body(double ds, Scalars *__restrict__ s
     for (int w = 1; w < NT / 64; ++w) {
         o[0] = fmax(o[0], red[w * 8 + 0]);
         o[1] = fmax(o[1], red[w * 8 + 1]);
-        for (int q = 2; q < 7; ++q) o[q] += red[w * 8 + q];
+        if (mode != 1)
+            for (int q = 2; q < 7; ++q) o[q] += red[w * 8 + q];
     }
     if (mode == 2) {
         for (int q = 0; q < 5; ++q) sc->sums[q] = o[2 + q];
         return;
     }
     if (mode == 1) {
-        if (!sc->active) return;
-        if constexpr (!BULK) sc->t = (double)(T(sc->t) + T(sc->dt));
-        else sc->t = sc->t + sc->dt;
-        sc->steps += 1;
+        if (!active) return;
+        if constexpr (!BULK) t_now = (double)(T(t_now) + T(dt_now));
+        else t_now = t_now + dt_now;
+        steps += 1;
+        sc->t = t_now;
+        sc->steps = steps;
     }
     const bool nan = o[1] != 0.0;
     double dt;
@@ -1473,7 +1512,7 @@ __device__ __forceinline__ void finalize_body(double ds, Scalars *__restrict__ s
     sc->maxden = o[0];
     if (mode == 0)
         for (int q = 0; q < 5; ++q) sc->sums[q] = o[2 + q];
-    sc->active = !((sc->t > sc->t_end) || (sc->steps >= sc->max_steps));
+    sc->active = !((t_now > t_end) || (steps >= max_steps));
 }
 
 template <typename T, bool BULK>
@@ -1626,8 +1665,7 @@ corr_flag_kernel(const StepArgs A, const Fields<float> U, float *__restrict__ B,
         }
     }
     if (!MASKED) {
-        const double nosums[5] = {0, 0, 0, 0, 0};
-        block_partials<256>((double)maxden, nanf, nosums, red, partials, blockIdx.x, threadIdx.x);
+        block_den<256>(maxden, nanf, red, partials + (size_t)blockIdx.x * PARTIAL_STRIDE, threadIdx.x);
     }
 }
 
@@ -1658,8 +1696,7 @@ corr_apply_kernel(const StepArgs A, const Fields<float> U, const float *__restri
         const float den = cell_den<float, FAST>(u, const_divisor(V, A.dV), 1.0f / V, gm1, gamma);
         if (den != den) nanf = 1; else maxden = fmaxf(maxden, den);
     }
-    const double nosums[5] = {0, 0, 0, 0, 0};
-    block_partials<256>((double)maxden, nanf, nosums, red, partials, blockIdx.x, threadIdx.x);
+    block_den<256>(maxden, nanf, red, partials + (size_t)blockIdx.x * PARTIAL_STRIDE, threadIdx.x);
 }
 
 // 2x restriction: coarse[I] = sum of the 8 children (U is extensive).
