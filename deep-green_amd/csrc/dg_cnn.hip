@@ -745,78 +745,95 @@ prep_target_kernel(const PrepArgs a, const float *const *__restrict__ samples, c
 // Divergence loss over the L^3 box: P[c][q] = -sum_d (G[c+1][5d+q] - G[c+1-e_d][5d+q])
 // (G on (L+1)^3, index c+1 = face c + e_d/2), loss = mean (P - T)^2 over cells and
 // the 5 components; dG = dloss/dG (bf16, 16 channels, channel 15 zero); per-block
-// partial loss sums.  A thread needs the errors of its cell and of three
-// neighbours, 40 16-byte loads (L1 and L2) and nothing to hide them but other
-// waves: 1024 threads per block.  8 crops of 32^3: 72 -> 36 us (scalar
-// loads, four errors per component, 256 threads).
-constexpr int LOSS_THREADS = 1024;
+// partial loss sums.
+// A face needs the errors of its cell and of three neighbours, each 15 loads
+// over 64-byte cells (the cache's tag rate bounds them), so they are computed
+// once: a workgroup takes a run of (y, z) positions of one batch item,
+// flattened, and marches a few x planes with the last planes' errors (its
+// positions and the Lg + 1 that follow them, the y and z neighbours) in LDS.
+// 8 crops of 32^3: 20 us; four errors per thread from memory, 36 us.
+constexpr int LOSS_THREADS = 512;
+constexpr int LOSS_EXT = 960;   // positions with errors per run: L up to 830 (a box of which needs 300 GB)
+struct LossGeom {
+    int run, nrun;     // positions per run, runs per plane
+    int cx, nxc;       // planes per item, items along x
+    long long items;   // B * nrun * nxc
+};
 __global__ void __launch_bounds__(LOSS_THREADS)
-loss_kernel(int B, int L, const float *__restrict__ G, const float *__restrict__ T, bf16 *__restrict__ dG,
-            double *__restrict__ loss_part)
+loss_kernel(int L, const LossGeom lg, double N, const float *__restrict__ G, const float *__restrict__ T,
+            bf16 *__restrict__ dG, double *__restrict__ loss_part)
 {
+    __shared__ float lds[3 * 5 * LOSS_EXT];
     __shared__ double red[LOSS_THREADS];
-    const int Lg = L + 1;
-    const uint32_t perg = (uint32_t)Lg * Lg * Lg;
-    const long long total = (long long)perg * B;
-    const double N = (double)B * L * L * L * 5;
+    const int Lg = L + 1, plane = Lg * Lg, ext = lg.run + Lg + 1, tid = threadIdx.x;
     const float scale = (float)(2.0 / N);
     double lsum = 0.0;
-    for (long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < total;
-         e += (long long)gridDim.x * blockDim.x) {
-        const int b = (int)(e / perg);
-        uint32_t r = (uint32_t)(e % perg);
-        const int gz = (int)(r % Lg); r /= Lg;
-        const int gy = (int)(r % Lg);
-        const int gx = (int)(r / Lg);
-        // errors of cell c (zero outside the box)
-        auto err = [&](int cx, int cy, int cz, float *out) {
-            if (cx < 0 || cy < 0 || cz < 0 || cx >= L || cy >= L || cz >= L) {
+    for (long long item = blockIdx.x; item < lg.items; item += gridDim.x) {
+        const int run = (int)(item % lg.nrun), xc = (int)(item / lg.nrun % lg.nxc);
+        const long long b = item / lg.nrun / lg.nxc;
+        const int p0 = run * lg.run, nown = min(lg.run, plane - p0), nerr = min(ext, plane - p0);
+        const int xs = xc * lg.cx, xe = min(xs + lg.cx, Lg);
+        // errors of the cells (cx, y - 1, z - 1) at positions p0 .. p0 + nerr - 1 (zero outside the box)
+        auto errors = [&](int cx) {
+            float *E = lds + (cx + 3) % 3 * 5 * ext;
+            for (int i = tid; i < nerr; i += LOSS_THREADS) {
+                const int gy = (p0 + i) / Lg, gz = (p0 + i) - gy * Lg;
+                float e[5] = {0, 0, 0, 0, 0};
+                if (cx >= 0 && cx < L && gy > 0 && gz > 0) {
+                    const f32x4 *own = reinterpret_cast<const f32x4 *>(
+                        G + ((b * Lg + cx + 1) * plane + p0 + i) * 16);
+                    const f32x4 *xm = own - (long long)plane * 4, *ym = own - (long long)Lg * 4, *zm = own - 4;
+                    const f32x4 a0 = own[0], a1 = own[1], a2 = own[2], a3 = own[3];
+                    const f32x4 x0 = xm[0], x1 = xm[1], y1 = ym[1], y2 = ym[2], z2 = zm[2], z3 = zm[3];
+                    const float gx0[5] = {a0[0], a0[1], a0[2], a0[3], a1[0]}, gx1[5] = {x0[0], x0[1], x0[2], x0[3], x1[0]};
+                    const float gy0[5] = {a1[1], a1[2], a1[3], a2[0], a2[1]}, gy1[5] = {y1[1], y1[2], y1[3], y2[0], y2[1]};
+                    const float gz0[5] = {a2[2], a2[3], a3[0], a3[1], a3[2]}, gz1[5] = {z2[2], z2[3], z3[0], z3[1], z3[2]};
+                    const float *t = T + (((b * L + cx) * L + gy - 1) * L + gz - 1) * 5;
 #pragma unroll
-                for (int q = 0; q < 5; ++q) out[q] = 0.0f;
-                return;
+                    for (int q = 0; q < 5; ++q)
+                        e[q] = -((gx0[q] - gx1[q]) + (gy0[q] - gy1[q]) + (gz0[q] - gz1[q])) - t[q];
+                }
+#pragma unroll
+                for (int q = 0; q < 5; ++q) E[q * ext + i] = e[q];
             }
-            const long long g0 = (long long)b * perg + (((long long)(cx + 1) * Lg + (cy + 1)) * Lg + (cz + 1));
-            const f32x4 *own = reinterpret_cast<const f32x4 *>(G + g0 * 16);
-            const f32x4 *xm = own - (long long)Lg * Lg * 4, *ym = own - (long long)Lg * 4, *zm = own - 4;
-            const f32x4 a0 = own[0], a1 = own[1], a2 = own[2], a3 = own[3];
-            const f32x4 x0 = xm[0], x1 = xm[1], y1 = ym[1], y2 = ym[2], z2 = zm[2], z3 = zm[3];
-            const float gx0[5] = {a0[0], a0[1], a0[2], a0[3], a1[0]}, gx1[5] = {x0[0], x0[1], x0[2], x0[3], x1[0]};
-            const float gy0[5] = {a1[1], a1[2], a1[3], a2[0], a2[1]}, gy1[5] = {y1[1], y1[2], y1[3], y2[0], y2[1]};
-            const float gz0[5] = {a2[2], a2[3], a3[0], a3[1], a3[2]}, gz1[5] = {z2[2], z2[3], z3[0], z3[1], z3[2]};
-            const float *t = T + ((((long long)b * L + cx) * L + cy) * L + cz) * 5;
-#pragma unroll
-            for (int q = 0; q < 5; ++q)
-                out[q] = -((gx0[q] - gx1[q]) + (gy0[q] - gy1[q]) + (gz0[q] - gz1[q])) - t[q];
         };
-        const int cx = gx - 1, cy = gy - 1, cz = gz - 1;
-        float e0[5], n[3][5];
-        err(cx, cy, cz, e0);
-        err(cx + 1, cy, cz, n[0]);
-        err(cx, cy + 1, cz, n[1]);
-        err(cx, cy, cz + 1, n[2]);
-        bf16x8 lo = zero8(), hi = zero8();
+        __syncthreads();   // the last item's reads are done
+        errors(xs - 1);
+        for (int gx = xs; gx < xe; ++gx) {
+            errors(gx);
+            __syncthreads();   // with three planes in LDS, the only one a plane needs
+            const float *E0 = lds + (gx + 2) % 3 * 5 * ext, *E1 = lds + gx % 3 * 5 * ext;
+            for (int i = tid; i < nown; i += LOSS_THREADS) {
+                const int gy = (p0 + i) / Lg, gz = (p0 + i) - gy * Lg;
+                bf16x8 lo = zero8(), hi = zero8();
 #pragma unroll
-        for (int q = 0; q < 5; ++q) {
-            if (cx >= 0 && cy >= 0 && cz >= 0) lsum += (double)e0[q] * e0[q];
-            // d/dG[g][5d+q]: -e(c) from cell c = g-1, + e(c + e_d) from cell g-1+e_d
+                for (int q = 0; q < 5; ++q) {
+                    const float e0 = E0[q * ext + i];
+                    lsum += (double)e0 * e0;   // (zero where there is no cell)
+                    // d/dG[g][5d+q]: -e(c) from cell c = g-1, + e(c + e_d) from cell g-1+e_d
+                    const float n[3] = {E1[q * ext + i], gy < L ? E0[q * ext + i + Lg] : 0.0f,
+                                        gz < L ? E0[q * ext + i + 1] : 0.0f};
 #pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                const int ch = 5 * d + q;
-                const bf16 v = (bf16)(scale * (-e0[q] + n[d][q]));
-                if (ch < 8) lo[ch] = v;
-                else hi[ch - 8] = v;
+                    for (int d = 0; d < 3; ++d) {
+                        const int ch = 5 * d + q;
+                        const bf16 v = (bf16)(scale * (-e0 + n[d]));
+                        if (ch < 8) lo[ch] = v;
+                        else hi[ch - 8] = v;
+                    }
+                }
+                bf16 *out = dG + ((b * Lg + gx) * plane + p0 + i) * 16;
+                *reinterpret_cast<bf16x8 *>(out) = lo;
+                *reinterpret_cast<bf16x8 *>(out + 8) = hi;
             }
         }
-        *reinterpret_cast<bf16x8 *>(dG + e * 16) = lo;
-        *reinterpret_cast<bf16x8 *>(dG + e * 16 + 8) = hi;
     }
-    red[threadIdx.x] = lsum;
+    red[tid] = lsum;
     __syncthreads();
     for (int s = LOSS_THREADS / 2; s > 0; s >>= 1) {
-        if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
+        if (tid < s) red[tid] += red[tid + s];
         __syncthreads();
     }
-    if (threadIdx.x == 0) loss_part[blockIdx.x] = red[0] / N;
+    if (tid == 0) loss_part[blockIdx.x] = red[0] / N;
 }
 
 // Host-array staging: fp32 [cells][creal] -> bf16 [cells][cpad]
@@ -1026,9 +1043,24 @@ int prep_target(const PrepArgs &a, const float *const *samples, const int *boxes
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
+// Runs of equal length whose errors one pass of the workgroup computes (longer
+// ones where a row alone is more), and items for the nblk workgroups.
 int loss(int B, int L, const float *G, const float *T, void *dG, double *loss_part, int nblk, hipStream_t s)
 {
-    hipLaunchKernelGGL(loss_kernel, dim3(nblk), dim3(LOSS_THREADS), 0, s, B, L, G, T, static_cast<bf16 *>(dG), loss_part);
+    const int Lg = L + 1, plane = Lg * Lg;
+    LossGeom lg;
+    const int fit = LOSS_THREADS - Lg - 1 > LOSS_THREADS / 4 ? LOSS_THREADS - Lg - 1 : LOSS_THREADS / 4;
+    lg.nrun = (plane + fit - 1) / fit;
+    lg.run = (plane + lg.nrun - 1) / lg.nrun;
+    const long long cols = (long long)B * lg.nrun;
+    long long nxc = (nblk + cols - 1) / cols;
+    if (nxc > Lg) nxc = Lg;
+    lg.cx = (int)((Lg + nxc - 1) / nxc);
+    lg.nxc = (Lg + lg.cx - 1) / lg.cx;
+    lg.items = cols * lg.nxc;
+    if (lg.run + Lg + 1 > LOSS_EXT) return -1;
+    hipLaunchKernelGGL(loss_kernel, dim3(nblk), dim3(LOSS_THREADS), 0, s, L, lg, (double)B * L * L * L * 5, G, T,
+                       static_cast<bf16 *>(dG), loss_part);
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 

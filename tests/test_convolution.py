@@ -92,3 +92,29 @@ def test_emulated_adam_packs_the_weights(emu_lib):  # noqa: F811
 @pytest.mark.gpu
 def test_adam_packs_the_weights():
     run_packed(None)
+
+
+def run_loss(lib, batch, L):
+    m = network(lib, 9)
+    rng = np.random.default_rng(L)
+    x = rng.normal(size=(batch, L + 7, L + 7, L + 7, 5)).astype(np.float32)
+    t = rng.normal(size=(batch, L, L, L, 5)).astype(np.float32)
+    loss, g = m.train_batch(x, t)
+    net = ref.Net(m.get_params())
+    want = ref.divergence_loss(net.forward(x), t)
+    want.backward()
+    assert abs(loss - want.item()) < 1e-2 * want.item()
+    check_grads(g, net.grads_flat())
+
+
+@pytest.mark.parametrize("batch,L", [(2, 1), (1, 4)])
+def test_emulated_loss_runs(emu_lib, batch, L):  # noqa: F811
+    run_loss(emu_lib, batch, L)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,L", [(1, 1), (3, 2), (40, 5), (2, 21), (1, 33), (9, 16)])
+def test_loss_runs(batch, L):
+    """One row to several runs of positions per plane, more and fewer items than workgroups."""
+    print(f"  loss {batch} x {L}^3", flush=True)
+    run_loss(None, batch, L)
