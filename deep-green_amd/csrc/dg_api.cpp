@@ -435,12 +435,16 @@ int reserve_partials(dg_ctx *c)
 }
 
 // One step (the step kernel, then dt / clock) on the context's stream.
-int launch_one_step(dg_ctx *c)
+// unbounded (no heat): whatever a dg_run left in the run clock, with the dt and
+// the step count to sc_host.
+static int one_step(dg_ctx *c, bool unbounded)
 {
     const void *in[5];
     void *out[5];
     for (int f = 0; f < 5; ++f) { in[f] = c->buf[c->cur][f]; out[f] = c->buf[1 - c->cur][f]; }
-    int rc = dg::launch_step(c->prec, c->fast, c->tile_y, c->args, in, out, c->sc, c->partials, c->stream);
+    StepArgs a = c->args;
+    if (unbounded) a.swizzle |= 2;
+    int rc = dg::launch_step(c->prec, c->fast, c->tile_y, a, in, out, c->sc, c->partials, c->stream);
     if (rc) return fail(c, DG_ERR_DEVICE, std::string("step launch: ") + hipGetErrorString(hipGetLastError()));
     int nparts = c->args.nblocks;
     if (c->heat_mask) {
@@ -454,12 +458,14 @@ int launch_one_step(dg_ctx *c)
         nparts = c->nparts_reduce;
     }
     rc = dg::launch_finalize(c->prec, c->args, c->sc, c->partials, nparts, c->cfg.cfl,
-                             c->cfg.dt_nan_fallback, 1, c->stream);
+                             c->cfg.dt_nan_fallback, 1, c->stream, unbounded ? c->sc_host : nullptr);
     if (rc) return fail(c, DG_ERR_DEVICE, "finalize launch");
     c->cur = 1 - c->cur;
     c->sums_stale = true;
     return DG_OK;
 }
+
+int launch_one_step(dg_ctx *c) { return one_step(c, false); }
 
 // Lift any stop condition of a previous dg_run (a step launched while the
 // scalars say "inactive" carries the state through unchanged).
@@ -666,16 +672,22 @@ int dg_step(dg_ctx *c, double *dt_used)
     if (!c) return DG_ERR_INVALID;
     if (!c->have_state) return fail(c, DG_ERR_STATE, "no state set");
     HIPCHK(c, hipSetDevice(c->cfg.device));
-    // arming also hands the host the dt, so one wait is enough; without the NaN
-    // fallback the dt decides whether there is a step.  30^3 FP32: 54 -> 43 us
-    // a call against arming, a copy of the scalars and two waits
-    arm(c, INFINITY, LLONG_MAX, 0, c->sc_host);
+    // The step ignores the run clock's bounds and its dt kernel lifts them and
+    // hands the host the dt: two launches and one wait (30^3 FP32: 43 ->
+    // 40 us a call against arming first).  Without the NaN fallback
+    // the dt decides whether there is a step, and heat reads the clock: armed.
     int rc;
-    if (!c->cfg.dt_nan_fallback) {
-        if ((rc = host_scalars(c))) return rc;
-        if (!std::isfinite(c->sc_host->dt)) return fail(c, DG_ERR_NONFINITE, "dt is not finite");
+    if (c->cfg.dt_nan_fallback && !c->heat_mask) {
+        c->sc_host->steps = -1;
+        if ((rc = dg::one_step(c, true))) return rc;
+    } else {
+        arm(c, INFINITY, LLONG_MAX, 0, c->sc_host);
+        if (!c->cfg.dt_nan_fallback) {
+            if ((rc = host_scalars(c))) return rc;
+            if (!std::isfinite(c->sc_host->dt)) return fail(c, DG_ERR_NONFINITE, "dt is not finite");
+        }
+        if ((rc = dg::launch_one_step(c))) return rc;
     }
-    if ((rc = dg::launch_one_step(c))) return rc;
     if ((rc = host_scalars(c))) return rc;
     if (dt_used) *dt_used = c->sc_host->dt;
     return DG_OK;

@@ -28,7 +28,8 @@ struct StepArgs {
     int lx;            // planes per workgroup along x
     int nbx, nby, nbz; // workgroups per axis
     int nblocks;
-    int swizzle;       // 1: spread tiles so each XCD works on a contiguous range
+    int swizzle;       // bit 0: spread tiles so each XCD works on a contiguous range; bit 1: step
+                       // whatever the run clock says
     int pow2;          // 1: ds is a power of two, so x / ds, x / (2 ds) and x / ds^3
                        //    equal the products with the exact reciprocals bit for bit
     double ds, gamma, g;
@@ -91,8 +92,11 @@ int launch_step(int prec, int fast, int tile_y, const StepArgs &a, const void *c
 int launch_reduce(int prec, int fast, const StepArgs &a, const void *const u[5], double *partials,
                   int nblocks, hipStream_t s);
 // mode 0: dt and sums of a fresh state; 1: after a step; 2: sums only
+// mode 0: a fresh state, 1: after a step, 2: sums only.  host (pinned, mode 1):
+// receives the dt the step used and the step count, and the run clock's bounds
+// are lifted.
 int launch_finalize(int prec, const StepArgs &a, Scalars *sc, const double *partials, int nparts,
-                    double cfl, int nan_fallback, int mode, hipStream_t s);
+                    double cfl, int nan_fallback, int mode, hipStream_t s, Scalars *host = nullptr);
 int launch_prim_to_cons(int prec, const StepArgs &a, void *const u[5], hipStream_t s);
 int launch_cons_to_prim(int prec, const StepArgs &a, const void *const u[5], void *const w[5],
                         hipStream_t s);
